@@ -267,6 +267,47 @@ def test_gdn2_prefill_device_block_widths(jt, orc, torch_cuda, H, T, C_, dk, dv)
         assert same(S1[h], Sh), h
 
 
+@pytest.mark.parametrize("H,T,C_,dk,dv", [
+    (1, 16, 16, 1, 5),      # one chunk, one value, a partial column group
+    (2, 64, 32, 31, 3), (1, 96, 32, 33, 259),   # around 2 blocks of 16 rows; two groups a block
+    (2, 64, 32, 97, 10), (1, 64, 32, 127, 7),   # 6 and 8 blocks with padded rows
+    (2, 48, 16, 64, 6), (1, 48, 16, 90, 1023),  # 4 and 6 blocks, C = 16
+    (1, 32, 16, 129, 9), (2, 48, 16, 250, 530)])  # 16 blocks
+def test_gdn2_prefill_device_row_blocks(jt, orc, torch_cuda, H, T, C_, dk, dv):
+    """Every row-block count of the state kernel at its edges, with ragged
+    columns, zero-norm rows, signed zeros and alphas of 0 and 1: bit for bit
+    the oracle's chunk chain (the tolerance is none: every chain keeps the
+    reference's order and roundings)."""
+    torch = torch_cuda
+    announce(f"jt_hip_gdn2_prefill row blocks H={H} T={T} C={C_} {dk}x{dv}")
+    rng = np.random.default_rng(dk * 3 + dv)
+    S = (rng.standard_normal((H, dk, dv)) * 0.3).astype(np.float32)
+    S[:, :, 0] = -0.0
+    Q, K, B = (rng.standard_normal((H, T, dk)).astype(np.float32) for _ in range(3))
+    A = rng.uniform(0.6, 1, (H, T, dk)).astype(np.float32)
+    A[:, 1, : dk // 2] = 1.0
+    A[:, T - 3, dk // 3:] = 0.0
+    Q[:, 2] = 0.0
+    K[:, 5] = 0.0
+    V, W = (rng.standard_normal((H, T, dv)).astype(np.float32) for _ in range(2))
+    V[:, :4, 0] = -0.0
+    W[:, 7] = 0.0
+    dS = _t(torch, S)
+    dOut = torch.empty((H, T, dv), device="cuda")
+    rc, _ = jt.gdn2_prefill_device(dS, dOut, *[_t(torch, x) for x in (Q, K, V, B, W, A)], C_)
+    assert rc == 0
+    assert jt.sync_errors() == 0
+    S1, O1 = dS.cpu().numpy(), dOut.cpu().numpy()
+    for h in range(H):
+        Sh = S[h]
+        for c0 in range(0, T, C_):
+            sl = slice(c0, c0 + C_)
+            rc, Sh, Oh = orc.gdn2_prefill_chunk(Sh, Q[h, sl], K[h, sl], V[h, sl], B[h, sl],
+                                                W[h, sl], A[h, sl])
+            assert rc == 0 and same(O1[h, sl], Oh), (h, c0)
+        assert same(S1[h], Sh), h
+
+
 def test_gdn2_prefill_full_size(jt, orc, torch_cuda):
     """The prefill benchmark's shape: 8 heads x 4096 tokens of 128x128
     states in chunks of 32, every head's state and every output against the
