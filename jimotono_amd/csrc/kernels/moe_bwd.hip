@@ -17,8 +17,9 @@
 //                 stable expert sort of the kept pairs
 // Expert path (steps 5-6): three bit-exact fp32 GEMM forms (per output, a
 // k-ascending sequence of rounded multiplies and rounded adds, as
-// src/moe_gemm.c:47-89) on 64x64 tiles:
-//  k_bwd_gemm<AT, BT, EPI> with EPI_DSWIGLU (dY Wd^T -> SwiGLU backward
+// src/moe_gemm.c:47-89), k_bwd_gemm_mx on 64x128 tiles for large layers,
+// k_bwd_gemm on smaller ones:
+//  <AT, BT, EPI> with EPI_DSWIGLU (dY Wd^T -> SwiGLU backward
 //  -> Dg, Du, S), EPI_DUAL ((float)((double)Dg Wg + (double)Du Wu)) and
 //  EPI_STORE (D^T X weight gradients).
 //  k_bwd_dx     : dX = (float)(gate + routed rows in perm order + shared)
@@ -109,17 +110,90 @@ struct Chunk {
 };
 
 // acc[i][j] += a[i] * b[j]: one rounded multiply, one rounded add
+template <int N>
+__device__ __forceinline__ void ld_row(float (&v)[N], const float *s) {
+    if constexpr (N % 4 == 0) {
+#pragma unroll
+        for (int i = 0; i < N; i += 4) *(float4 *)&v[i] = *(const float4 *)(s + i);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; i += 2) *(float2 *)&v[i] = *(const float2 *)(s + i);
+    }
+}
 template <int TM, int TN>
 __device__ __forceinline__ void mul_add(float (&acc)[TM][TN], const float *as, const float *bs) {
     float av[TM], bv[TN];
-#pragma unroll
-    for (int i = 0; i < TM; i += 4) *(float4 *)&av[i] = *(const float4 *)(as + i);
-#pragma unroll
-    for (int j = 0; j < TN; j += 4) *(float4 *)&bv[j] = *(const float4 *)(bs + j);
+    ld_row(av, as);
+    ld_row(bv, bs);
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++) acc[i][j] = __fadd_rn(acc[i][j], __fmul_rn(av[i], bv[j]));
+}
+
+// What a block computes: rows rb .. rb+rc, columns cb .. cb+cc of group g
+// (matrix m) on one side, K products from A, B. False: nothing.
+struct Job {
+    int side, g, m, rb, rc, cb, cc, K;
+    const float *A[2], *B[2];
+};
+template <int EPI, int MODE, int BM, int BN>
+__device__ __forceinline__ bool gemm_job(const GemmP &p, Job &j) {
+    j.m = 0;
+    if (MODE == MODE_ROWS) {
+        const int bx = blockIdx.x;
+        if (bx < p.nsh) {
+            j.side = 0, j.g = bx / p.mt_sh, j.rb = (bx % p.mt_sh) * BM;
+            j.rc = min(BM, p.sd[0].M - j.rb);
+        } else {
+            j.side = 1;
+            if (bx - p.nsh >= *p.sd[1].ntiles) return false;
+            const int4 tl = p.sd[1].tiles[bx - p.nsh];
+            j.g = tl.x, j.rb = tl.y, j.rc = tl.z;
+        }
+    } else {
+        int z = blockIdx.z;
+        j.side = z < p.nsh ? 0 : 1;
+        z -= j.side ? p.nsh : 0;
+        j.g = z / 3, j.m = z % 3;
+        j.rb = blockIdx.x * BM;
+        j.rc = min(BM, p.sd[j.side].M - j.rb);
+    }
+    const Side &S = p.sd[j.side];
+    j.cb = blockIdx.y * BN, j.cc = min(BN, p.N - j.cb);
+    j.K = S.K;
+    int64_t kb = 0;
+    if (MODE == MODE_WGRAD && S.koff) {
+        kb = S.koff[j.g];
+        j.K = S.koff[j.g + 1] - S.koff[j.g];
+    }
+    j.A[0] = S.A[j.m] + j.g * S.sAg + kb * S.sAk;
+    j.B[0] = S.B[j.m] + j.g * S.sBg + kb * S.sBk;
+    j.A[1] = EPI == EPI_DUAL ? S.A[1] + j.g * S.sAg + kb * S.sAk : j.A[0];
+    j.B[1] = EPI == EPI_DUAL ? S.B[1] + j.g * S.sBg + kb * S.sBk : j.B[0];
+    return true;
+}
+// Output (r, c) of the block from its sums; false when not finite
+template <int EPI>
+__device__ __forceinline__ bool gemm_out(const Side &S, const Job &j, int r, int c, float acc,
+                                         float acc2) {
+    const int64_t row = j.rb + r, col = j.cb + c;
+    const int64_t o = j.g * S.sCg + row * S.ldc + col;
+    if constexpr (EPI == EPI_STORE) {
+        S.C[j.m][o] = acc;
+    } else if constexpr (EPI == EPI_DUAL) {
+        S.C[0][o] = (float)((double)acc + (double)acc2);
+    } else {
+        const int64_t q = S.rowq ? S.rowq[row] : row;
+        const int64_t at = j.g * S.sGg + q * S.ldg + col;
+        float dg, du, sv;
+        const bool ok = dswiglu(S.G[at], S.U[at], acc, &dg, &du, &sv);
+        S.C[0][o] = dg;
+        S.C[1][o] = du;
+        S.C[2][o] = sv;
+        return ok;
+    }
+    return true;
 }
 
 template <bool AT, bool BT, int EPI, int MODE, int TM, int TN>
@@ -129,40 +203,11 @@ __global__ __launch_bounds__(256) void k_bwd_gemm(GemmP p) {
     __shared__ __attribute__((aligned(16))) float As[NP][BK][BM + PAD];
     __shared__ __attribute__((aligned(16))) float Bs[NP][BK][BN + PAD];
     const int tid = threadIdx.x;
-    int side, g, m = 0, rb, rc;
-    if (MODE == MODE_ROWS) {
-        const int bx = blockIdx.x;
-        if (bx < p.nsh) {
-            side = 0, g = bx / p.mt_sh, rb = (bx % p.mt_sh) * BM;
-            rc = min(BM, p.sd[0].M - rb);
-        } else {
-            side = 1;
-            if (bx - p.nsh >= *p.sd[1].ntiles) return;
-            const int4 tl = p.sd[1].tiles[bx - p.nsh];
-            g = tl.x, rb = tl.y, rc = tl.z;
-        }
-    } else {
-        int z = blockIdx.z;
-        side = z < p.nsh ? 0 : 1;
-        z -= side ? p.nsh : 0;
-        g = z / 3, m = z % 3;
-        rb = blockIdx.x * BM;
-        rc = min(BM, p.sd[side].M - rb);
-    }
-    const Side &S = p.sd[side];
-    const int cb = blockIdx.y * BN, cc = min(BN, p.N - cb);
-    int K = S.K;
-    int64_t kb = 0;
-    if (MODE == MODE_WGRAD && S.koff) {
-        kb = S.koff[g];
-        K = S.koff[g + 1] - S.koff[g];
-    }
-    const float *Ag = S.A[m] + g * S.sAg + kb * S.sAk, *Bg = S.B[m] + g * S.sBg + kb * S.sBk;
-    const float *Ag2 = Ag, *Bg2 = Bg;
-    if (EPI == EPI_DUAL) {
-        Ag2 = S.A[1] + g * S.sAg + kb * S.sAk;
-        Bg2 = S.B[1] + g * S.sBg + kb * S.sBk;
-    }
+    Job j;
+    if (!gemm_job<EPI, MODE, BM, BN>(p, j)) return;
+    const Side &S = p.sd[j.side];
+    const float *Ag = j.A[0], *Bg = j.B[0], *Ag2 = j.A[1], *Bg2 = j.B[1];
+    const int rb = j.rb, rc = j.rc, cb = j.cb, cc = j.cc, K = j.K;
     const int ty = tid / 16, tx = tid % 16;
     float acc[TM][TN], acc2[EPI == EPI_DUAL ? TM : 1][EPI == EPI_DUAL ? TN : 1];
 #pragma unroll
@@ -218,40 +263,122 @@ __global__ __launch_bounds__(256) void k_bwd_gemm(GemmP p) {
         }
         __syncthreads();
     }
-    bool bad = false;
+    bool ok = true;
 #pragma unroll
     for (int i = 0; i < TM; i++) {
         const int r = ty * TM + i;
         if (r >= rc) continue;
-        const int64_t row = rb + r;
-        const int64_t o = g * S.sCg + row * S.ldc;
-        const int64_t q = (EPI == EPI_DSWIGLU && S.rowq) ? S.rowq[row] : row;
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int c = tx * TN + j;
+        for (int jc = 0; jc < TN; jc++) {
+            const int c = tx * TN + jc;
             if (c >= cc) continue;
-            const int col = cb + c;
-            if constexpr (EPI == EPI_STORE) {
-                S.C[m][o + col] = acc[i][j];
-            } else if constexpr (EPI == EPI_DUAL) {
-                S.C[0][o + col] = (float)((double)acc[i][j] + (double)acc2[i][j]);
-            } else {
-                const int64_t at = g * S.sGg + q * S.ldg + col;
-                float dg, du, sv;
-                bad |= !dswiglu(S.G[at], S.U[at], acc[i][j], &dg, &du, &sv);
-                S.C[0][o + col] = dg;
-                S.C[1][o + col] = du;
-                S.C[2][o + col] = sv;
-            }
+            float a2 = 0.0f;
+            if constexpr (EPI == EPI_DUAL) a2 = acc2[i][jc];
+            ok &= gemm_out<EPI>(S, j, r, c, acc[i][jc], a2);
         }
     }
-    if (bad) raise_err(p.err, EF_NONFINITE_MID);
+    if (!ok) raise_err(p.err, EF_NONFINITE_MID);
 }
 
-template <bool AT, bool BT, int EPI, int MODE, int TM, int TN>
-int launch_gemm(const GemmP &p, dim3 grid, hipStream_t s) {
-    if (grid.x == 0 || grid.y == 0 || grid.z == 0) return 0;
-    hipLaunchKernelGGL((k_bwd_gemm<AT, BT, EPI, MODE, TM, TN>), grid, dim3(256), 0, s, p);
+typedef float v32f __attribute__((ext_vector_type(32)));
+
+// The same sums on 64 x 128 tiles with the products made by the matrix
+// cores: v_mfma_f32_32x32x1 with a zero accumulator gives 32 x 64 rounded
+// products of one k (a product of -0 comes out as +0, which changes no sum:
+// a sum that starts from +0 is never -0), the adds stay on the VALU. fp32
+// MFMA and VALU share the lanes' multipliers, so the bound is that of a
+// multiply and an add per product (147 cycles of a SIMD for 2048 measured,
+// 149 with v_mul and v_add, 33.7 T products/s on the chip). What it saves is
+// everything around: one 4-byte LDS read of A and of B per lane and k for
+// 2048 products, where 4 x 4 outputs a thread read 32 bytes for 1024.
+// The two products of EPI_DUAL run one after the other.
+template <bool AT, bool BT, int EPI, int MODE>
+__global__ __launch_bounds__(256, EPI == EPI_DUAL ? 2 : 3) void k_bwd_gemm_mx(GemmP p) {
+    constexpr int BM = 64, BN = 128, BK = 16;
+    constexpr int NP = EPI == EPI_DUAL ? 2 : 1;
+    __shared__ float As[BK][BM + PAD], Bs[BK][BN + PAD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    Job j;
+    if (!gemm_job<EPI, MODE, BM, BN>(p, j)) return;
+    const Side &S = p.sd[j.side];
+    const int wm = wave >> 1, wn = wave & 1, K = j.K;  // wave tile 32 x 64
+    v32f acc[NP];
+#pragma unroll
+    for (int pr = 0; pr < NP; pr++) {
+        v32f sum = {};
+        Chunk<BM, BK, AT> ca;
+        Chunk<BN, BK, !BT> cb;
+        if (K > 0) {
+            ca.load(j.A[pr], S.lda, j.rb, j.rc, 0, K, tid);
+            cb.load(j.B[pr], S.ldb, j.cb, j.cc, 0, K, tid);
+        }
+        const float *ap = &As[0][wm * 32 + (lane & 31)], *bp = &Bs[0][wn * 64 + lane];
+        auto step = [&](int kk) {
+            const v32f zero = {};
+            sum = sum + __builtin_amdgcn_mfma_f32_32x32x1f32(ap[kk * (BM + PAD)],
+                                                             bp[kk * (BN + PAD)], zero, 1, 0, 0);
+        };
+        for (int k0 = 0; k0 < K; k0 += BK) {
+            ca.store(As, tid);
+            cb.store(Bs, tid);
+            __syncthreads();
+            if (k0 + BK < K) {  // the next chunk's loads overlap this chunk's products
+                ca.load(j.A[pr], S.lda, j.rb, j.rc, k0 + BK, K, tid);
+                cb.load(j.B[pr], S.ldb, j.cb, j.cc, k0 + BK, K, tid);
+            }
+            if (K - k0 >= BK) {
+#pragma unroll
+                for (int kk = 0; kk < BK; kk++) step(kk);
+            } else {
+                for (int kk = 0; kk < K - k0; kk++) step(kk);
+            }
+            __syncthreads();
+        }
+        acc[pr] = sum;
+    }
+    bool ok = true;
+#pragma unroll
+    for (int v = 0; v < 32; v++) {
+        const int r = wm * 32 + (v & 15) / 4 * 8 + (lane >> 5) * 4 + (v & 3);
+        const int c = wn * 64 + (v >> 4) * 32 + (lane & 31);
+        if (r < j.rc && c < j.cc) ok &= gemm_out<EPI>(S, j, r, c, acc[0][v], acc[NP - 1][v]);
+    }
+    if (!ok) raise_err(p.err, EF_NONFINITE_MID);
+}
+
+// rows: row tiles of 64 (MODE_ROWS, both sides) or output rows
+// (MODE_WGRAD); groups: grid z; many: no serial sum is long beside the whole
+// launch. The matrix-core form from 1024 tiles of 64 x 128 on, where it has
+// two waves or more on a SIMD (4096 tokens, n 1024, h 256, 64 experts top-8
+// and one shared: 481, 900 and 1164 us against 541, 977 and 1237 with 4 x 4
+// outputs a thread); a step of its sum takes 400 cycles, so a shared expert's
+// K = T must not outlast the rest (`many`; n 512, h 256, 32 experts top-4 and
+// one shared at T = 4096: 687 us against 469 with 2 x 4). Below that a block's
+// time is its serial K loop and small tiles are faster (64 tokens of the first
+// layer, 146 and 584 tiles: 104 and 147 us with 4 x 2 outputs a thread, 137
+// and 151 with 4 x 4, 162 and 168 in the matrix-core form; 27 tiles of weight
+// gradients with K = 512: 30 us with 2 x 2, 47 with 2 x 4, 63 with 4 x 4).
+template <bool AT, bool BT, int EPI, int MODE>
+int launch_gemm(const GemmP &p, unsigned rows, unsigned groups, bool many, hipStream_t s) {
+    if (rows == 0 || p.N <= 0 || groups == 0) return 0;
+    auto grid = [&](int BM, int BN) {
+        return dim3(MODE == MODE_ROWS ? rows : (rows + BM - 1) / BM,
+                    (unsigned)((p.N + BN - 1) / BN), groups);
+    };
+    const dim3 g = grid(64, 128);
+    const int64_t tiles = (int64_t)g.x * g.y * g.z;
+    if (tiles >= 1024 && many) {
+        hipLaunchKernelGGL((k_bwd_gemm_mx<AT, BT, EPI, MODE>), g, dim3(256), 0, s, p);
+    } else if constexpr (MODE == MODE_ROWS) {
+        hipLaunchKernelGGL((k_bwd_gemm<AT, BT, EPI, MODE, 4, 2>), grid(64, 32), dim3(256), 0, s,
+                           p);
+    } else if (tiles >= 64) {
+        hipLaunchKernelGGL((k_bwd_gemm<AT, BT, EPI, MODE, 2, 4>), grid(32, 64), dim3(256), 0, s,
+                           p);
+    } else {
+        hipLaunchKernelGGL((k_bwd_gemm<AT, BT, EPI, MODE, 2, 2>), grid(32, 32), dim3(256), 0, s,
+                           p);
+    }
     return (int)hipGetLastError();
 }
 
@@ -378,42 +505,87 @@ __global__ __launch_bounds__(256) void k_bwd_gather(const uint64_t *__restrict__
     }
 }
 
-// dw[q] for every pair, 0 for dropped ones.
+__device__ __forceinline__ float quad_xor1(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                                                 0xB1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float quad_xor2(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                                                 0x4E, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double quad_xor1(double x) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0xB1, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0xB1, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ double quad_xor2(double x) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, 0x4E, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x4E, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// v.x .. v.w of the quad's four lanes -> x[i] = element (lane & 3) of lane i
+__device__ __forceinline__ void quad_transpose(float4 v, int lq, float (&x)[4]) {
+    float s0 = lq & 1 ? v.x : v.y, s1 = lq & 1 ? v.z : v.w;
+    s0 = quad_xor1(s0), s1 = quad_xor1(s1);
+    const float y0 = lq & 1 ? s0 : v.x, y1 = lq & 1 ? v.y : s0;
+    const float y2 = lq & 1 ? s1 : v.z, y3 = lq & 1 ? v.w : s1;
+    float u0 = lq & 2 ? y0 : y2, u1 = lq & 2 ? y1 : y3;
+    u0 = quad_xor2(u0), u1 = quad_xor2(u1);
+    x[0] = lq & 2 ? u0 : y0, x[1] = lq & 2 ? u1 : y1;
+    x[2] = lq & 2 ? y2 : u0, x[3] = lq & 2 ? y3 : u1;
+}
+
+// dw[q] for every pair, 0 for dropped ones. Four lanes a pair, one for each
+// of the sum's four chains over j % 4; with n % 16 == 0 and aligned rows the
+// quad reads 64 bytes of a row at a time and transposes them so that lane c
+// has the next four values of chain c (products of two floats are exact in
+// fp64, so the fused step rounds as the separate one). Bound by reading Ysel:
+// 134 MB at 4096 tokens x top-8, n 1024 (a thread a pair, each lane on its own
+// row: 83 us).
 __global__ __launch_bounds__(256) void k_bwd_dots(const float *__restrict__ Ysel,
                                                   const float *__restrict__ dY,
                                                   const uint8_t *__restrict__ drop, int Tk,
                                                   int k, int n, double *__restrict__ dw,
                                                   uint32_t *err) {
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= Tk) return;
-    if (drop[q]) {
+    const int q = blockIdx.x * 64 + (threadIdx.x >> 2), lq = threadIdx.x & 3;
+    const bool live = q < Tk && !drop[q];
+    const float *y = Ysel + (int64_t)q * n, *d = dY + (int64_t)(q / k) * n;
+    double l = 0.0;
+    const int n4 = n & ~3;
+    if ((n & 15) == 0 && (((uintptr_t)Ysel | (uintptr_t)dY) & 15) == 0) {
+        const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        for (int j0 = 0; j0 < n; j0 += 64) {  // 4 steps' loads ahead of the sums
+            float4 a[4], b[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int j = j0 + 16 * u + 4 * lq;
+                a[u] = live && j < n ? *(const float4 *)(y + j) : zero;
+                b[u] = live && j < n ? *(const float4 *)(d + j) : zero;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                float x[4], z[4];
+                quad_transpose(a[u], lq, x);
+                quad_transpose(b[u], lq, z);
+#pragma unroll
+                for (int i = 0; i < 4; i++) l = fma((double)x[i], (double)z[i], l);
+            }
+        }
+    } else if (live) {
+        for (int j = lq; j < n4; j += 4) l = l + (double)y[j] * (double)d[j];
+    }
+    l = l + quad_xor1(l);  // (l0 + l1) + (l2 + l3), in all four lanes
+    l = l + quad_xor2(l);
+    if (q >= Tk || lq != 0) return;
+    if (!live) {
         dw[q] = 0.0;
         return;
     }
-    const float *y = Ysel + (int64_t)q * n, *d = dY + (int64_t)(q / k) * n;
-    double l0 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
-    const int n4 = n & ~3;
-    int j = 0;
-    if ((n & 3) == 0) {
-        for (; j < n4; j += 4) {
-            const float4 a = *(const float4 *)(y + j), b = *(const float4 *)(d + j);
-            l0 = l0 + (double)a.x * (double)b.x;
-            l1 = l1 + (double)a.y * (double)b.y;
-            l2 = l2 + (double)a.z * (double)b.z;
-            l3 = l3 + (double)a.w * (double)b.w;
-        }
-    } else {
-        for (; j < n4; j += 4) {
-            l0 = l0 + (double)y[j] * (double)d[j];
-            l1 = l1 + (double)y[j + 1] * (double)d[j + 1];
-            l2 = l2 + (double)y[j + 2] * (double)d[j + 2];
-            l3 = l3 + (double)y[j + 3] * (double)d[j + 3];
-        }
-    }
-    double s = (l0 + l1) + (l2 + l3);
-    for (; j < n; j++) s = s + (double)y[j] * (double)d[j];
-    if (!isfinite(s)) raise_err(err, EF_NONFINITE_MID);
-    dw[q] = s;
+    for (int j = n4; j < n; j++) l = l + (double)y[j] * (double)d[j];
+    if (!isfinite(l)) raise_err(err, EF_NONFINITE_MID);
+    dw[q] = l;
 }
 
 // Per token: s = sum_kept (double)w*dw in slot order; dlog[q] =
@@ -482,34 +654,44 @@ __global__ __launch_bounds__(256) void k_bwd_token(
 
 // dWgate[e][j] = float sum over the kept pairs of expert e in flattened
 // index order of (float)(dlog*(double)X[t][j]); 0 for experts without one.
-// The pairs are read 16 at a time ahead of the (ordered) sums.
-__global__ __launch_bounds__(256) void k_bwd_dwgate(const int32_t *__restrict__ off2,
-                                                    const int32_t *__restrict__ perm2,
-                                                    const double *__restrict__ dlog,
-                                                    const float *__restrict__ X, int k, int n,
-                                                    float *__restrict__ dWgate) {
-    const int e = blockIdx.x, j = blockIdx.y * 256 + threadIdx.x;
-    if (j >= n) return;
+// 64 columns a block; the pairs' rows and dlog go through LDS 256 at a time,
+// and 32 rows' values are loaded ahead of the (ordered) sums, so a batch costs
+// one load latency, not the three of pair, dlog and row (4096 tokens x top-8,
+// 64 experts, n 1024: 65 us with 16 rows a batch from global indices).
+__global__ __launch_bounds__(64) void k_bwd_dwgate(const int32_t *__restrict__ off2,
+                                                   const int32_t *__restrict__ perm2,
+                                                   const double *__restrict__ dlog,
+                                                   const float *__restrict__ X, int k, int n,
+                                                   float *__restrict__ dWgate) {
+    __shared__ int rows[256];
+    __shared__ double dls[256];
+    const int e = blockIdx.x, j = blockIdx.y * 64 + threadIdx.x, jc = min(j, n - 1);
     float rg = 0.0f;
     const int i0 = off2[e], i1 = off2[e + 1];
-    int i = i0;
-    for (; i + 16 <= i1; i += 16) {
-        float x[16];
-        double dl[16];
+    for (int b = i0; b < i1; b += 256) {
+        const int m = min(256, i1 - b);
+        __syncthreads();
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int q = perm2[i + u];
-            dl[u] = dlog[q];
-            x[u] = X[(int64_t)(q / k) * n + j];
+        for (int u = 0; u < 256; u += 64) {
+            const int i = u + threadIdx.x;
+            if (i < m) {
+                const int q = perm2[b + i];
+                rows[i] = q / k;
+                dls[i] = dlog[q];
+            }
         }
+        __syncthreads();
+        int i = 0;
+        for (; i + 32 <= m; i += 32) {
+            float x[32];
 #pragma unroll
-        for (int u = 0; u < 16; u++) rg = rg + (float)(dl[u] * (double)x[u]);
+            for (int u = 0; u < 32; u++) x[u] = X[(int64_t)rows[i + u] * n + jc];
+#pragma unroll
+            for (int u = 0; u < 32; u++) rg = rg + (float)(dls[i + u] * (double)x[u]);
+        }
+        for (; i < m; i++) rg = rg + (float)(dls[i] * (double)X[(int64_t)rows[i] * n + jc]);
     }
-    for (; i < i1; i++) {
-        const int q = perm2[i];
-        rg = rg + (float)(dlog[q] * (double)X[(int64_t)(q / k) * n + j]);
-    }
-    dWgate[(int64_t)e * n + j] = rg;
+    if (j < n) dWgate[(int64_t)e * n + j] = rg;
 }
 
 // dX[t][j] = (float)(0 + gate term + routed rows in ascending perm order +
@@ -537,10 +719,7 @@ __global__ __launch_bounds__(256) void k_bwd_dx(
 
 inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
 
-// Tile shapes (threads hold TM x TN outputs; blocks 16 TM x 16 TN). The row
-// GEMMs share one routed tile list, so they share TM.
-constexpr int TM_ROWS = 4, TN_DOT = 4, TN_DX = 4, TM_WG = 4, TN_WG = 4;
-constexpr int BM_ROWS = 16 * TM_ROWS;
+constexpr int BM_ROWS = 64;  // rows of a routed tile
 
 }  // namespace
 
@@ -634,7 +813,7 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
     }
     // gate path
     if (io->dLogits) le |= jtk_zero_u32((uint32_t *)io->dLogits, (int64_t)T * E, s);
-    hipLaunchKernelGGL(k_bwd_dots, dim3(cdiv(Tk, 256)), dim3(256), 0, s, io->Ysel, io->dY,
+    hipLaunchKernelGGL(k_bwd_dots, dim3(cdiv(Tk, 64)), dim3(256), 0, s, io->Ysel, io->dY,
                        io->drop, Tk, k, n, w->dw, err);
     hipLaunchKernelGGL(k_bwd_token, dim3(cdiv(T, 256)), dim3(256), 0, s, io->ids, io->weights,
                        io->drop, w->dw, w->inv, T, k, E, w->dlog, io->dLogits, w->gate_e,
@@ -642,7 +821,7 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
     le |= (int)hipGetLastError();
     le |= jtk_sort(w->key, Tk, E + 1, (int64_t)Tk, w->rank, w->cnt, w->tot, w->off2, nullptr,
                    w->perm2, nullptr, nullptr, err, s);
-    hipLaunchKernelGGL(k_bwd_dwgate, dim3((unsigned)E, cdiv(n, 256)), dim3(256), 0, s, w->off2,
+    hipLaunchKernelGGL(k_bwd_dwgate, dim3((unsigned)E, cdiv(n, 64)), dim3(64), 0, s, w->off2,
                        w->perm2, w->dlog, io->X, k, n, io->dWgate);
     // expert rows in perm order
     hipLaunchKernelGGL(k_bwd_gather, dim3((unsigned)Tk), dim3(256), 0, s, io->perm, io->X,
@@ -669,8 +848,7 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
         b.G = io->Gsel, b.U = io->Usel, b.rowq = w->rowq, b.ldg = h;
         b.K = n, b.tiles = (const int4 *)w->tiles, b.ntiles = w->ntiles;
     }
-    le |= launch_gemm<false, true, EPI_DSWIGLU, MODE_ROWS, TM_ROWS, TN_DOT>(
-        p, dim3(p.nsh + mt, cdiv(h, 16 * TN_DOT)), s);
+    le |= launch_gemm<false, true, EPI_DSWIGLU, MODE_ROWS>(p, p.nsh + mt, 1, true, s);
     // dx rows = (float)((double)(Dg Wg) + (double)(Du Wu))
     p = GemmP{};
     p.err = err, p.N = n, p.nsh = S * mt_sh, p.mt_sh = mt_sh;
@@ -686,8 +864,7 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
         b.C[0] = w->Dxe, b.ldc = n;
         b.K = h, b.tiles = (const int4 *)w->tiles, b.ntiles = w->ntiles;
     }
-    le |= launch_gemm<false, false, EPI_DUAL, MODE_ROWS, TM_ROWS, TN_DX>(
-        p, dim3(p.nsh + mt, cdiv(n, 16 * TN_DX)), s);
+    le |= launch_gemm<false, false, EPI_DUAL, MODE_ROWS>(p, p.nsh + mt, 1, true, s);
     // weight gradients D^T rows: dWg = Dg^T X, dWu = Du^T X, dWd = S^T dY
     // (routed: weighted dY rows, over the expert's rows in perm order)
     p = GemmP{};
@@ -704,8 +881,10 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
         b.C[0] = io->dWg, b.C[1] = io->dWu, b.C[2] = io->dWd, b.ldc = n, b.sCg = nh;
         b.M = h, b.koff = w->off32;
     }
-    le |= launch_gemm<true, false, EPI_STORE, MODE_WGRAD, TM_WG, TN_WG>(
-        p, dim3(cdiv(h, 16 * TM_WG), cdiv(n, 16 * TN_WG), (unsigned)(3 * (S + E))), s);
+    // a tile's sum over the T tokens of a shared expert against all tiles'
+    // sums, 400 cycles a step and 0.33 ns a step of the whole chip
+    const bool many = S == 0 || 3LL * (S + k) * cdiv(h, 64) * cdiv(n, 128) >= 400;
+    le |= launch_gemm<true, false, EPI_STORE, MODE_WGRAD>(p, h, 3 * (S + E), many, s);
     hipLaunchKernelGGL(k_bwd_dx, dim3((unsigned)T, cdiv(n, 256)), dim3(256), 0, s, io->Wgate,
                        w->gate_e, w->gate_dl, w->gate_n, w->tokpos, w->tokcnt, w->Dxe, w->SDxe,
                        S, T, k, n, io->dX, err);

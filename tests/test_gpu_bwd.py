@@ -103,6 +103,24 @@ def test_bwd_vs_oracle(jt, orc, case):
             assert np.array_equal(bits(u[nm]), bits(o[nm])), nm
 
 
+@pytest.mark.parametrize("case", [
+    (300, 136, 130, 520, 2, 1, 21, None),   # matrix-core form in all three products
+    (70, 260, 68, 530, 3, 0, 22, 1.0),      # no shared experts, one column tile of 68
+    (130, 48, 40, 12, 2, 1, 23, None)])     # the smallest tiles, K = 130 of the shared expert
+def test_bwd_tile_forms_vs_oracle(jt, orc, case):
+    """The product forms at ragged tiles: 64 x 128 with products from the
+    matrix cores (1024 tiles and more), 4 x 2, 2 x 4 and 2 x 2 outputs a
+    thread below. Every form keeps the order and the two roundings, so the
+    bounds are check()'s."""
+    announce(f"moe_bwd_batch tile forms {case}")
+    c = bwd_case(*case)
+    want = orc.moe_bwd_batch(*bwd_args(c))
+    assert want["rc"] == 0
+    o = jt.moe_bwd_batch(*bwd_args(c))
+    assert o["rc"] == 0
+    check(o, want, label=str(case))
+
+
 def test_bwd_without_logits(jt, orc):
     announce("moe_bwd_batch dLogits NULL")
     c = bwd_case(20, 40, 24, 6, 2, 1, 31, 1.0)
