@@ -3,9 +3,10 @@
 //  k_router_logits : logits[t][e] = (float)dot(X[t], Wgate[e]) in fp64 with
 //                    the reference's four lane partials over j % 4, combined
 //                    as (l0+l1)+(l2+l3), then the tail (src/moe_layer.c:67-86,
-//                    1118-1137). Products of two floats are exact in fp64, so
-//                    fma(x, w, l) rounds exactly like the reference's
-//                    separate multiply and add.
+//                    1118-1137), on fp64 matrix cores, beside the tokens'
+//                    codes. Products of two floats are exact in fp64, so a
+//                    fused step rounds exactly like the reference's separate
+//                    multiply and add.
 //  k_topk          : top-k by value with ties to the lower index, softmax
 //                    over the selected k in fp64 (src/routing.c:16-76).
 //  k_sort_*        : stable counting sort of the (token, slot) pairs by
@@ -14,19 +15,42 @@
 //                    fp64, slot order then shared order
 //                    (src/moe_layer.c:1443-1463, 1549-1574).
 #include "jt_dev.h"
+#include "gemm_w8a8.h"
 #include "jt_launch.h"
 #include "topk_dev.h"
 #include "sort_dev.h"
 #include "quant_dev.h"
 
 // ---------------- router logits ----------------
-// Block: 64 tokens x 64 experts, 256 threads in 4 groups of 64; group p
-// accumulates the reference's lane partial l_p = sum over j = p (mod 4) of
-// x_j*w_j (j ascending) for all 64 x 64 outputs, each thread an 8 x 8
-// (token, expert) register tile of fp64 accumulators. K is staged through
-// LDS as fp32, k-major, in chunks of 32 (double-buffered). At the end the
-// partials meet in LDS and are combined as (l0+l1)+(l2+l3), then the tail
-// j >= n & ~3 is added in order, as in the reference.
+// Every logit exact, on the fp64 matrix cores: v_mfma_f64_16x16x4 adds its
+// four products to an accumulator one after the other, k ascending, each a
+// fused multiply-add (checked bit for bit against that chain), so with the
+// four k values of an instruction at j, j + 4, j + 8, j + 12 it runs four
+// steps of one of the reference's lane partials (j = p mod 4) for 16 tokens x
+// 16 experts. The partials meet as (l0+l1)+(l2+l3), then the tail
+// j >= n & ~3 is added in order. Lane l holds row l % 16 of both operands, k
+// value l / 16; element i of its result is token 4 i + l / 16, expert l % 16.
+// (Values past n & ~3 are zeros, which change no sum: a partial starts from
+// +0 and is never -0.)
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// the tail and the store of one logit; false when it is not finite
+__device__ __forceinline__ bool logit_out(const float *X, const float *Wg, int T, int E, int n,
+                                          int t, int e, double v, float *logits) {
+    if (t >= T || e >= E) return true;
+    for (int j = n & ~3; j < n; j++)
+        v = v + (double)X[(int64_t)t * n + j] * (double)Wg[(int64_t)e * n + j];
+    const float f = (float)v;
+    logits[(int64_t)t * E + e] = f;
+    return isfinite(v) && isfinite(f);
+}
+
+// Block: 64 tokens x 64 experts, 4 waves, wave p the lane partial l_p of all
+// 64 x 64 outputs as 4 x 4 matrix tiles. K is staged through LDS widened to
+// fp64, k-major, in chunks of 32 (double-buffered), and chunks go out to
+// registers four ahead, since a chunk's products take a load's latency only.
+// 1531 tokens x 512 experts, n 2048: 114 us on 192 blocks (145 with v_fma on
+// 8 x 8 outputs a thread, 140 with the next chunk alone in flight).
 #define RT_T 64
 #define RT_E 64
 #define RT_KC 32
@@ -40,88 +64,100 @@ __global__ __launch_bounds__(256) void k_router_logits(const float *__restrict__
     __shared__ __attribute__((aligned(16))) double lds[2][2][RT_KC][64];
     const int tid = threadIdx.x;
     const int t0 = blockIdx.x * RT_T, e0 = blockIdx.y * RT_E;
-    const int p = tid >> 6;                       // lane partial of this thread
-    const int ty = (tid >> 3) & 7, tx = tid & 7;  // tokens ty*8.., experts tx*8..
-    double acc[8][8];
+    const int p = tid >> 6;                        // lane partial of this wave
+    const int lane = tid & 63, r = lane & 15, kq = lane >> 4;
+    v4d acc[4][4];  // [16 tokens][16 experts]
 #pragma unroll
-    for (int a = 0; a < 8; a++)
+    for (int a = 0; a < 4; a++)
 #pragma unroll
-        for (int b = 0; b < 8; b++) acc[a][b] = 0.0;
+        for (int b = 0; b < 4; b++) acc[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
     const int n4 = n & ~3;
-    // stage loader: thread -> row tid%64, k = 8*(tid/64) .. +7 of the chunk;
+    // stage loader (zeros past n4): thread -> row tid%64, k = 8*(tid/64) .. +7 of the chunk;
     // LDS stores of consecutive threads are consecutive (no bank conflicts)
     const int lr = tid & 63, lk = (tid >> 6) * 8;
     const float *xrow = X + (int64_t)min(t0 + lr, T - 1) * n;
     const float *wrow = Wg + (int64_t)min(e0 + lr, E - 1) * n;
     const bool vec = (n & 3) == 0;
-    float xv[8], wv[8];
-    auto gload = [&](int k0) {
+    constexpr int PF = 4;  // chunks in registers on their way to LDS
+    float xv[PF][8], wv[PF][8];
+    auto gload = [&](int k0, float (&x)[8], float (&w)[8]) {
         const int kb = k0 + lk;
         if (vec && kb + 8 <= n4) {
             const float4 a0 = *(const float4 *)(xrow + kb), a1 = *(const float4 *)(xrow + kb + 4);
             const float4 b0 = *(const float4 *)(wrow + kb), b1 = *(const float4 *)(wrow + kb + 4);
-            xv[0] = a0.x; xv[1] = a0.y; xv[2] = a0.z; xv[3] = a0.w;
-            xv[4] = a1.x; xv[5] = a1.y; xv[6] = a1.z; xv[7] = a1.w;
-            wv[0] = b0.x; wv[1] = b0.y; wv[2] = b0.z; wv[3] = b0.w;
-            wv[4] = b1.x; wv[5] = b1.y; wv[6] = b1.z; wv[7] = b1.w;
+            x[0] = a0.x; x[1] = a0.y; x[2] = a0.z; x[3] = a0.w;
+            x[4] = a1.x; x[5] = a1.y; x[6] = a1.z; x[7] = a1.w;
+            w[0] = b0.x; w[1] = b0.y; w[2] = b0.z; w[3] = b0.w;
+            w[4] = b1.x; w[5] = b1.y; w[6] = b1.z; w[7] = b1.w;
         } else {
 #pragma unroll
             for (int c = 0; c < 8; c++) {
                 const int k = kb + c;
-                xv[c] = k < n4 ? xrow[k] : 0.0f;
-                wv[c] = k < n4 ? wrow[k] : 0.0f;
+                x[c] = k < n4 ? xrow[k] : 0.0f;
+                w[c] = k < n4 ? wrow[k] : 0.0f;
             }
         }
     };
-    auto sstore = [&](int buf) {
+    auto sstore = [&](int buf, const float (&x)[8], const float (&w)[8]) {
 #pragma unroll
         for (int c = 0; c < 8; c++) {
-            lds[buf][0][lk + c][lr] = (double)xv[c];
-            lds[buf][1][lk + c][lr] = (double)wv[c];
+            lds[buf][0][lk + c][lr] = (double)x[c];
+            lds[buf][1][lk + c][lr] = (double)w[c];
         }
     };
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < n4; k0 += RT_KC) {
-        const bool more = k0 + RT_KC < n4;
-        if (more) gload(k0 + RT_KC);
-        const int kend = min(RT_KC, n4 - k0);
-        for (int i = p; i < kend; i += 4) {
-            double xa[8], wa[8];
+    auto chunk = [&](int buf) {
 #pragma unroll
-            for (int c = 0; c < 8; c += 2) {
-                const double2 xx = *(const double2 *)&lds[buf][0][i][ty * 8 + c];
-                const double2 ww = *(const double2 *)&lds[buf][1][i][tx * 8 + c];
-                xa[c] = xx.x;
-                xa[c + 1] = xx.y;
-                wa[c] = ww.x;
-                wa[c + 1] = ww.y;
+        for (int i = 0; i < RT_KC; i += 16) {
+            double xa[4], wa[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                xa[c] = lds[buf][0][i + 4 * kq + p][16 * c + r];
+                wa[c] = lds[buf][1][i + 4 * kq + p][16 * c + r];
             }
 #pragma unroll
-            for (int a = 0; a < 8; a++)
+            for (int a = 0; a < 4; a++)
 #pragma unroll
-                for (int b = 0; b < 8; b++) acc[a][b] = fma(xa[a], wa[b], acc[a][b]);
+                for (int b = 0; b < 4; b++)
+                    acc[a][b] =
+                        __builtin_amdgcn_mfma_f64_16x16x4f64(xa[a], wa[b], acc[a][b], 0, 0, 0);
         }
-        if (more) sstore(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
+    };
+    static_assert(PF % 2 == 0, "LDS buffer = chunk parity");
+#pragma unroll
+    for (int u = 0; u < PF; u++) gload(u * RT_KC, xv[u], wv[u]);
+    sstore(0, xv[0], wv[0]);
+    lds_barrier();
+    for (int k0 = 0; k0 < n4; k0 += PF * RT_KC) {
+#pragma unroll
+        for (int u = 0; u < PF; u++) {
+            const int k = k0 + u * RT_KC;
+            if (k >= n4) break;
+            // slot u was stored with the chunk before; refill it
+            gload(k + PF * RT_KC, xv[u], wv[u]);
+            chunk(u & 1);
+            if (k + RT_KC < n4) sstore((u + 1) & 1, xv[(u + 1) % PF], wv[(u + 1) % PF]);
+            lds_barrier();
+        }
     }
     // combine partials through LDS (reusing the staging arrays):
     // l1 -> l0+l1, l3 -> l2+l3, then (l0+l1)+(l2+l3)
-    double *red = &lds[0][0][0][0];
+    double *red = &lds[0][0][0][0] + lane;
     auto put = [&]() {
 #pragma unroll
-        for (int a = 0; a < 8; a++)
+        for (int a = 0; a < 4; a++)
 #pragma unroll
-            for (int b = 0; b < 8; b++) red[(ty * 8 + a) * 64 + tx * 8 + b] = acc[a][b];
+            for (int b = 0; b < 4; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) red[((a * 4 + b) * 4 + i) * 64] = acc[a][b][i];
     };
     auto add = [&]() {
 #pragma unroll
-        for (int a = 0; a < 8; a++)
+        for (int a = 0; a < 4; a++)
 #pragma unroll
-            for (int b = 0; b < 8; b++) acc[a][b] = acc[a][b] + red[(ty * 8 + a) * 64 + tx * 8 + b];
+            for (int b = 0; b < 4; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    acc[a][b][i] = acc[a][b][i] + red[((a * 4 + b) * 4 + i) * 64];
     };
     if (p == 1) put();
     __syncthreads();
@@ -135,30 +171,94 @@ __global__ __launch_bounds__(256) void k_router_logits(const float *__restrict__
     __syncthreads();
     if (p != 0) return;
     add();
-    uint32_t bad = 0;
+    bool bad = false;
 #pragma unroll
-    for (int a = 0; a < 8; a++) {
-        const int t = t0 + ty * 8 + a;
-        if (t >= T) continue;
+    for (int a = 0; a < 4; a++)
 #pragma unroll
-        for (int b = 0; b < 8; b++) {
-            const int e = e0 + tx * 8 + b;
-            if (e >= E) continue;
-            double s = acc[a][b];
-            for (int j = n4; j < n; j++)
-                s = s + (double)X[(int64_t)t * n + j] * (double)Wg[(int64_t)e * n + j];
-            const float f = (float)s;
-            bad |= (!isfinite(s)) || (!isfinite(f));
-            logits[(int64_t)t * E + e] = f;
+        for (int b = 0; b < 4; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                bad |= !logit_out(X, Wg, T, E, n, t0 + 16 * a + 4 * i + kq, e0 + 16 * b + r,
+                                  acc[a][b][i], logits);
+    if (__ballot(bad) && lane == 0) raise_err(err, EF_NONFINITE_MID);
+}
+
+
+// One 16 x 16 tile a block, a partial to each wave, for token and expert
+// counts that leave 64 x 64 tiles few: operands straight from memory (16 rows
+// x 64 bytes a step), 16 steps' loads in flight while 16 are summed.
+__global__ __launch_bounds__(256) void k_router_logits_tile(const float *__restrict__ X,
+                                                            const float *__restrict__ Wg, int T,
+                                                            int E, int n,
+                                                            float *__restrict__ logits,
+                                                            uint32_t *err) {
+    __shared__ double part[3][4][64];
+    const int lane = threadIdx.x & 63;
+    const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int te = (E + 15) / 16, t0 = blockIdx.x / te * 16, e0 = blockIdx.x % te * 16;
+    const int r = lane & 15, kq = lane >> 4, n4 = n & ~3;
+    const float *xr = X + (int64_t)min(t0 + r, T - 1) * n;
+    const float *wr = Wg + (int64_t)min(e0 + r, E - 1) * n;
+    constexpr int D = 16;
+    v4d acc = {0.0, 0.0, 0.0, 0.0};
+    float xa[2][D], wa[2][D];
+    // a batch's loads go out together: past n4 the address stays in the row
+    // (n >= 4 whenever there is a step) and the value is replaced
+    auto load = [&](int s0, int b) {
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int j = min(16 * (s0 + d) + 4 * kq + p, n4 - 4 + p);
+            xa[b][d] = xr[j];
+            wa[b][d] = wr[j];
         }
+    };
+    auto sums = [&](int s0, int b) {
+        if (16 * (s0 + D) > n4) {
+#pragma unroll
+            for (int d = 0; d < D; d++)
+                if (16 * (s0 + d) + 4 * kq >= n4) xa[b][d] = wa[b][d] = 0.0f;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int d = 0; d < D; d++)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xa[b][d], (double)wa[b][d], acc, 0,
+                                                       0, 0);
+    };
+    const int ns = (n4 + 15) / 16;
+    if (ns > 0) load(0, 0);
+    for (int s0 = 0; s0 < ns; s0 += 2 * D) {
+        load(s0 + D, 1);
+        sums(s0, 0);
+        if (s0 + D >= ns) break;
+        load(s0 + 2 * D, 0);
+        sums(s0 + D, 1);
     }
-    if (bad) raise_err(err, EF_NONFINITE_MID);
+    if (p > 0)
+#pragma unroll
+        for (int i = 0; i < 4; i++) part[p - 1][i][lane] = acc[i];
+    __syncthreads();
+    if (p > 0) return;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        bad |= !logit_out(X, Wg, T, E, n, t0 + 4 * i + kq, e0 + r,
+                          (acc[i] + part[0][i][lane]) + (part[1][i][lane] + part[2][i][lane]),
+                          logits);
+    if (__ballot(bad) && lane == 0) raise_err(err, EF_NONFINITE_MID);
 }
 
 extern "C" int jtk_router_logits(const float *X, const float *Wg, int T, int E, int n,
                                  float *logits, uint32_t *err, hipStream_t s) {
-    dim3 grid((unsigned)((T + RT_T - 1) / RT_T), (unsigned)((E + RT_E - 1) / RT_E));
-    hipLaunchKernelGGL(k_router_logits, grid, dim3(256), 0, s, X, Wg, T, E, n, logits, err);
+    const int64_t tiles = (int64_t)((T + 15) / 16) * ((E + 15) / 16);
+    // (512 experts, n 2048: 256 tokens, 512 tiles: the layer 410 us against 463
+    // with 64 x 64 tiles; 1024 tokens: 732 against 607)
+    if (tiles < 1024) {
+        hipLaunchKernelGGL(k_router_logits_tile, dim3((unsigned)tiles), dim3(256), 0, s, X, Wg, T,
+                           E, n, logits, err);
+    } else {
+        dim3 grid((unsigned)((T + RT_T - 1) / RT_T), (unsigned)((E + RT_E - 1) / RT_E));
+        hipLaunchKernelGGL(k_router_logits, grid, dim3(256), 0, s, X, Wg, T, E, n, logits, err);
+    }
     return (int)hipGetLastError();
 }
 

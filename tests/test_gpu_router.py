@@ -144,3 +144,38 @@ def test_router_decode_all_exact(jt, orc, torch_cuda, T, n, E, k):
     check(orc, X, Wgate, k, ids, w, lg)
     rc, _, _, olg = orc.router(X, Wgate, k)
     assert np.array_equal(bits(lg), bits(olg))
+
+
+@pytest.mark.parametrize("T,n,E,k", [(17, 256, 300, 4),    # E past 256: 16 x 16 tiles
+                                     (37, 512, 257, 8),    # ragged tiles both ways
+                                     (900, 256, 300, 8)])  # 64 x 64 tiles, ragged
+def test_router_exact_logits_many_experts(jt, orc, torch_cuda, T, n, E, k):
+    """Layers beyond the bound router's 256 experts: every logit comes from
+    the fp64 matrix cores and must equal the reference's to the bit."""
+    announce(f"router exact logits T={T} n={n} E={E}")
+    rng = np.random.default_rng(T + n)
+    X = (rng.standard_normal((T, n)) * 10.0 ** rng.integers(-3, 4, (T, 1))).astype(np.float32)
+    X[0, :7] = -0.0
+    Wgate = (rng.standard_normal((E, n)) / np.sqrt(n)).astype(np.float32)
+    ids, w, lg = route(jt, torch_cuda, X, Wgate, k)
+    check(orc, X, Wgate, k, ids, w, lg)
+    assert np.array_equal(bits(lg), bits(orc.router(X, Wgate, k)[3]))
+
+
+@pytest.mark.parametrize("T,n,E", [(5, 1, 9), (9, 3, 17), (40, 70, 20), (33, 18, 40),
+                                   (900, 39, 290)])
+def test_router_logits_any_width(jt, orc, T, n, E):
+    """The host-pointer forward's logits at widths that are no multiple of the
+    matrix cores' four k values: the tail j >= n & ~3, partial steps."""
+    announce(f"router logits width T={T} n={n} E={E}")
+    rng = np.random.default_rng(n)
+    f = np.float32
+    X = rng.standard_normal((T, n)).astype(f)
+    Wgate = rng.standard_normal((E, n)).astype(f)
+    W = [(rng.standard_normal((E, 4, n)) / 2).astype(f) for _ in range(3)]
+    a = jt.moe_fwd_batch(X, Wgate, *W, None, None, None, 3, 1.5)
+    b = orc.moe_fwd_batch(X, Wgate, *W, None, None, None, 3, 1.5)
+    assert a["rc"] == 0 and b["rc"] == 0
+    assert np.array_equal(a["ids"], b["ids"])
+    # (the softmax's exp is within an ulp of glibc's: as the layer tests)
+    np.testing.assert_allclose(a["w"], b["w"], rtol=1e-6, atol=0)
