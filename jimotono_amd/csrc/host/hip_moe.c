@@ -762,9 +762,14 @@ static int moe_forward(jt_hip_moe *L, const float *dX, const int32_t *d_ids,
      * the codes, 0.332-0.334 forking after the approximate logits) */
     const int fork_late = fork && fast;
     if (fork && !fork_late) le |= fork_shared(L, T, fused, err, s);
-    /* 16-row tiles when experts average at most 16 rows; the single-launch
-     * sort up to 1024 pairs */
-    const int R = Tk <= 16 * E ? 16 : 64;
+    /* 16-row tiles when experts average at most 16 rows and either the
+     * one-launch FFN of such tiles takes the shape or the tiles are few: the
+     * generic 16-row kernel costs about 0.6 us a tile (512 experts, n 2048,
+     * h 512, one shared expert: 8 tokens 72 us against 83 with 64-row tiles, 16
+     * tokens 122 against 119, 64 tokens 224 against 181, 1024 tokens 585
+     * against 337) */
+    const int ffn16 = h == 256 && n % 256 == 0 && n <= 1024;
+    const int R = Tk <= 16 * E && (ffn16 || (Tk < E ? Tk : E) < 128) ? 16 : 64;
     /* tiles: at most Tk / R plus one per expert that holds a pair */
     const int max_tiles = Tk / R + (E < Tk ? E : Tk);
     /* Decode with the shared experts concatenated: top-k, the pair sort and
@@ -841,7 +846,7 @@ static int moe_forward(jt_hip_moe *L, const float *dX, const int32_t *d_ids,
         }
     }
     prof_mark(L, slot, ST_R_GATEUP, s);
-    if (R == 16 && h == 256 && n % 256 == 0 && n <= 1024) {
+    if (R == 16 && ffn16) {
         /* 16-row tiles: gate/up, SwiGLU, row codes and down in one launch
          * (the three stages are timed as one, under routed_gateup) */
         if (qsort_gu)

@@ -179,3 +179,20 @@ def test_router_logits_any_width(jt, orc, T, n, E):
     assert np.array_equal(a["ids"], b["ids"])
     # (the softmax's exp is within an ulp of glibc's: as the layer tests)
     np.testing.assert_allclose(a["w"], b["w"], rtol=1e-6, atol=0)
+
+
+def test_routed_tile_height_same_rows(jt, torch_cuda):
+    """Experts of 512 hidden rows take 64-row tiles from 128 tiles on and
+    16-row ones below: a token's output does not depend on it."""
+    torch = torch_cuda
+    announce("routed tile heights")
+    n, h, E, k, T = 256, 512, 160, 8, 40
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    L = jt.MoE(n, h, E, k, 0, 0, T, rn(E, n), rn(E, h, n) / 16, rn(E, h, n) / 16,
+               rn(E, h, n) / 22)
+    X = rn(T, n)
+    Y, Y8 = torch.empty_like(X), torch.empty(8, n, device="cuda")
+    assert L.fwd(X, Y) == 0 and L.fwd(X[:8].contiguous(), Y8) == 0
+    assert jt.sync_errors() == 0
+    assert np.array_equal(bits(Y[:8].cpu().numpy()), bits(Y8.cpu().numpy()))
