@@ -382,7 +382,8 @@ int launch_gemm(const GemmP &p, unsigned rows, unsigned groups, bool many, hipSt
     return (int)hipGetLastError();
 }
 
-// Finiteness of up to 16 arrays in one launch (blockIdx.y = array).
+// Finiteness of up to 16 arrays in one launch (blockIdx.y = array); HBM bound
+// (450 MB at 4096 tokens, n 1024: 85 us, 120 with one load in flight).
 struct FinList {
     const float *p[16];
     int64_t n[16];
@@ -395,6 +396,13 @@ __global__ __launch_bounds__(256) void k_bwd_finite(FinList L, uint32_t *err) {
     const int64_t step = (int64_t)gridDim.x * 256;
     if (((uintptr_t)x & 15) == 0) {  // float4 body
         const float4 *x4 = (const float4 *)x;
+        for (; i + 3 * step < n / 4; i += 4 * step) {  // four loads in flight
+            const float4 a = x4[i], b = x4[i + step], c = x4[i + 2 * step], d = x4[i + 3 * step];
+            bad |= !isfinite(a.x) || !isfinite(a.y) || !isfinite(a.z) || !isfinite(a.w);
+            bad |= !isfinite(b.x) || !isfinite(b.y) || !isfinite(b.z) || !isfinite(b.w);
+            bad |= !isfinite(c.x) || !isfinite(c.y) || !isfinite(c.z) || !isfinite(c.w);
+            bad |= !isfinite(d.x) || !isfinite(d.y) || !isfinite(d.z) || !isfinite(d.w);
+        }
         for (; i < n / 4; i += step) {
             const float4 v = x4[i];
             bad |= !isfinite(v.x) || !isfinite(v.y) || !isfinite(v.z) || !isfinite(v.w);
@@ -499,9 +507,20 @@ __global__ __launch_bounds__(256) void k_bwd_gather(const uint64_t *__restrict__
     const int64_t t = q / k;
     const double wv = (double)w[q];
     if (threadIdx.x == 0) rowq[i] = q;
+    const float *x = X + t * n, *d = dY + t * n;
+    float *xp = Xp + (int64_t)i * n, *dp = dYp + (int64_t)i * n;
+    if ((n & 3) == 0 && (((uintptr_t)X | (uintptr_t)dY) & 15) == 0) {
+        for (int j = threadIdx.x; j < n / 4; j += 256) {
+            const float4 a = ((const float4 *)x)[j], b = ((const float4 *)d)[j];
+            ((float4 *)xp)[j] = a;
+            ((float4 *)dp)[j] = make_float4((float)(wv * (double)b.x), (float)(wv * (double)b.y),
+                                            (float)(wv * (double)b.z), (float)(wv * (double)b.w));
+        }
+        return;
+    }
     for (int j = threadIdx.x; j < n; j += 256) {
-        Xp[(int64_t)i * n + j] = X[t * n + j];
-        dYp[(int64_t)i * n + j] = (float)(wv * (double)dY[t * n + j]);
+        xp[j] = x[j];
+        dp[j] = (float)(wv * (double)d[j]);
     }
 }
 
@@ -542,8 +561,8 @@ __device__ __forceinline__ void quad_transpose(float4 v, int lq, float (&x)[4]) 
 // quad reads 64 bytes of a row at a time and transposes them so that lane c
 // has the next four values of chain c (products of two floats are exact in
 // fp64, so the fused step rounds as the separate one). Bound by reading Ysel:
-// 134 MB at 4096 tokens x top-8, n 1024 (a thread a pair, each lane on its own
-// row: 83 us).
+// 134 MB at 4096 tokens x top-8, n 1024: 47 us (74 without the next 64 values in
+// flight; a thread a pair, each lane on its own row: 83).
 __global__ __launch_bounds__(256) void k_bwd_dots(const float *__restrict__ Ysel,
                                                   const float *__restrict__ dY,
                                                   const uint8_t *__restrict__ drop, int Tk,
@@ -556,22 +575,31 @@ __global__ __launch_bounds__(256) void k_bwd_dots(const float *__restrict__ Ysel
     const int n4 = n & ~3;
     if ((n & 15) == 0 && (((uintptr_t)Ysel | (uintptr_t)dY) & 15) == 0) {
         const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        for (int j0 = 0; j0 < n; j0 += 64) {  // 4 steps' loads ahead of the sums
-            float4 a[4], b[4];
+        float4 a[2][4], b[2][4];
+        auto load = [&](int j0, int p) {
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const int j = j0 + 16 * u + 4 * lq;
-                a[u] = live && j < n ? *(const float4 *)(y + j) : zero;
-                b[u] = live && j < n ? *(const float4 *)(d + j) : zero;
+                a[p][u] = live && j < n ? *(const float4 *)(y + j) : zero;
+                b[p][u] = live && j < n ? *(const float4 *)(d + j) : zero;
             }
+        };
+        auto sums = [&](int p) {
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 float x[4], z[4];
-                quad_transpose(a[u], lq, x);
-                quad_transpose(b[u], lq, z);
+                quad_transpose(a[p][u], lq, x);
+                quad_transpose(b[p][u], lq, z);
 #pragma unroll
                 for (int i = 0; i < 4; i++) l = fma((double)x[i], (double)z[i], l);
             }
+        };
+        load(0, 0);
+        for (int j0 = 0; j0 < n; j0 += 128) {  // the next 64 values in flight
+            load(j0 + 64, 1);
+            sums(0);
+            load(j0 + 128, 0);
+            sums(1);
         }
     } else if (live) {
         for (int j = lq; j < n4; j += 4) l = l + (double)y[j] * (double)d[j];
@@ -657,7 +685,7 @@ __global__ __launch_bounds__(256) void k_bwd_token(
 // 64 columns a block; the pairs' rows and dlog go through LDS 256 at a time,
 // and 32 rows' values are loaded ahead of the (ordered) sums, so a batch costs
 // one load latency, not the three of pair, dlog and row (4096 tokens x top-8,
-// 64 experts, n 1024: 65 us with 16 rows a batch from global indices).
+// 64 experts, n 1024: 32 us, 65 with 16 rows a batch from global indices).
 __global__ __launch_bounds__(64) void k_bwd_dwgate(const int32_t *__restrict__ off2,
                                                    const int32_t *__restrict__ perm2,
                                                    const double *__restrict__ dlog,
@@ -702,19 +730,50 @@ __global__ __launch_bounds__(256) void k_bwd_dx(
     const int32_t *__restrict__ tokpos, const int32_t *__restrict__ tokcnt,
     const float *__restrict__ Dxe, const float *__restrict__ SDxe, int S, int T, int k, int n,
     float *__restrict__ dX, uint32_t *err) {
-    const int t = blockIdx.x, j = blockIdx.y * 256 + threadIdx.x;
-    if (j >= n) return;
-    double acc = 0.0;
-    const int nk = gate_n[t];
-    for (int a = 0; a < nk; a++)
-        acc = acc + gate_dl[2 * t + a] * (double)Wgate[(int64_t)gate_e[2 * t + a] * n + j];
-    double dx = 0.0;
-    dx = dx + acc;
-    const int c = tokcnt[t];
-    for (int u = 0; u < c; u++) dx = dx + (double)Dxe[(int64_t)tokpos[(int64_t)t * k + u] * n + j];
-    for (int s = 0; s < S; s++) dx = dx + (double)SDxe[((int64_t)s * T + t) * n + j];
-    if (!isfinite(dx)) raise_err(err, EF_NONFINITE_MID);
-    dX[(int64_t)t * n + j] = (float)dx;
+    const int t = blockIdx.x, nk = gate_n[t], c = tokcnt[t];
+    const int32_t *pos = tokpos + (int64_t)t * k;
+    if ((n & 3) == 0 && (((uintptr_t)Wgate | (uintptr_t)dX) & 15) == 0) {
+        // four columns a thread with 16-byte loads
+        const int j = blockIdx.y * 256 + threadIdx.x;
+        if (4 * j >= n) return;
+        double acc[4] = {}, dx[4] = {};
+        auto add = [](double (&s)[4], double m, float4 v) {
+            s[0] = s[0] + m * (double)v.x, s[1] = s[1] + m * (double)v.y;
+            s[2] = s[2] + m * (double)v.z, s[3] = s[3] + m * (double)v.w;
+        };
+        auto row = [&](const float *p, int64_t r) { return ((const float4 *)(p + r * n))[j]; };
+        for (int a = 0; a < nk; a++)
+            add(acc, gate_dl[2 * t + a], row(Wgate, gate_e[2 * t + a]));
+#pragma unroll
+        for (int i = 0; i < 4; i++) dx[i] = dx[i] + acc[i];
+        int u = 0;
+        for (; u + 4 <= c; u += 4) {  // four rows in flight
+            float4 v[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q] = row(Dxe, pos[u + q]);
+#pragma unroll
+            for (int q = 0; q < 4; q++) add(dx, 1.0, v[q]);
+        }
+        for (; u < c; u++) add(dx, 1.0, row(Dxe, pos[u]));
+        for (int s = 0; s < S; s++) add(dx, 1.0, row(SDxe, (int64_t)s * T + t));
+        if (!isfinite(dx[0]) || !isfinite(dx[1]) || !isfinite(dx[2]) || !isfinite(dx[3]))
+            raise_err(err, EF_NONFINITE_MID);
+        ((float4 *)(dX + (int64_t)t * n))[j] =
+            make_float4((float)dx[0], (float)dx[1], (float)dx[2], (float)dx[3]);
+        return;
+    }
+    // one column a thread (blockIdx.y walks n / 4 columns' worth of threads)
+    for (int j = blockIdx.y * 256 + threadIdx.x; j < n; j += gridDim.y * 256) {
+        double acc = 0.0;
+        for (int a = 0; a < nk; a++)
+            acc = acc + gate_dl[2 * t + a] * (double)Wgate[(int64_t)gate_e[2 * t + a] * n + j];
+        double dx = 0.0;
+        dx = dx + acc;
+        for (int u = 0; u < c; u++) dx = dx + (double)Dxe[(int64_t)pos[u] * n + j];
+        for (int s = 0; s < S; s++) dx = dx + (double)SDxe[((int64_t)s * T + t) * n + j];
+        if (!isfinite(dx)) raise_err(err, EF_NONFINITE_MID);
+        dX[(int64_t)t * n + j] = (float)dx;
+    }
 }
 
 inline unsigned cdiv(int64_t a, int64_t b) { return (unsigned)((a + b - 1) / b); }
@@ -885,7 +944,7 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
     // sums, 400 cycles a step and 0.33 ns a step of the whole chip
     const bool many = S == 0 || 3LL * (S + k) * cdiv(h, 64) * cdiv(n, 128) >= 400;
     le |= launch_gemm<true, false, EPI_STORE, MODE_WGRAD>(p, h, 3 * (S + E), many, s);
-    hipLaunchKernelGGL(k_bwd_dx, dim3((unsigned)T, cdiv(n, 256)), dim3(256), 0, s, io->Wgate,
+    hipLaunchKernelGGL(k_bwd_dx, dim3((unsigned)T, cdiv(n, 1024)), dim3(256), 0, s, io->Wgate,
                        w->gate_e, w->gate_dl, w->gate_n, w->tokpos, w->tokcnt, w->Dxe, w->SDxe,
                        S, T, k, n, io->dX, err);
     le |= (int)hipGetLastError();
