@@ -539,8 +539,8 @@ __device__ __forceinline__ float solve16(float x, const float4 (&m)[4], int tt) 
 // by instruction latency: of 4700 cycles, phase 1 takes 2000 (128 steps of
 // two instructions, 9.7 cycles), the two solves 900, phase 3 800, LDS round
 // trips and barriers the rest. 8 heads x 4096 tokens of 128x128 in chunks of
-// 32: 256 us (k_gdn2_cols4, a thread per column for the solve and four
-// barriers a chunk: 1142 us).
+// 32: 256 us (with a thread per column for the solve and four barriers a
+// chunk: 1142 us).
 __host__ __device__ constexpr int scan_threads(int C, int NSUB) {
     return 64 * NSUB * (C / 8 + 2);
 }
