@@ -30,10 +30,12 @@ int jt_hip_gdn2_decode(float *dS, float *dO, const float *dq, const float *dk_,
 /* Heads per prefill call: the heads are a grid dimension of its launches. */
 #define JT_HIP_GDN2_MAX_PREFILL_HEADS 65535
 
-/* Workspace bytes of jt_hip_gdn2_prefill (0 for invalid arguments, H
- * outside 1..JT_HIP_GDN2_MAX_PREFILL_HEADS included):
+/* Workspace bytes for jt_hip_gdn2_prefill at full speed (0 for invalid
+ * arguments, H outside 1..JT_HIP_GDN2_MAX_PREFILL_HEADS included):
  * 4*ceil(H/64)*64 + H*(T/C)*(7*C*dk + 2*C*C)*4 -- one record per (head,
- * chunk), since every chunk's state-independent part is prepared at once. */
+ * chunk), since every chunk's state-independent part is prepared at once --
+ * and more than that for dk <= 22 (C = 16) and dk <= 13 (C = 32), where the
+ * fast kernels' records are padded. */
 size_t jt_hip_gdn2_prefill_ws_bytes(int H, int T, int C, int dk);
 /* Prefill of T tokens per head in T/C chunks of C = 16 or 32 (T % C == 0),
  * each chunk equal to the reference's jt_gdn2_prefill_chunk{C} on the state
@@ -41,7 +43,8 @@ size_t jt_hip_gdn2_prefill_ws_bytes(int H, int T, int C, int dk);
  * S [H][dk][dv] in place. A head with a bad value among its T tokens keeps
  * its S and Out. H in 1..JT_HIP_GDN2_MAX_PREFILL_HEADS (JT_ERR_INVAL,
  * EINVAL otherwise). d_ws: jt_hip_gdn2_prefill_ws_bytes(H, T, C, dk) bytes,
- * 16-byte aligned, not kept between calls. */
+ * 16-byte aligned, not kept between calls; from the formula's size on a
+ * smaller one is taken too, with the same results, a little more slowly. */
 int jt_hip_gdn2_prefill(float *dS, float *dOut, const float *dQ,
                         const float *dK, const float *dV, const float *dB,
                         const float *dW, const float *dA, int H, int T, int C,

@@ -146,14 +146,15 @@ static int prefill_chunk(float *S, float *Out, const float *Q, const float *K, c
     jt_rt *rt = jt_rt_get();
     if (!rt) return JT_ERR_IO;
     const size_t sb = (size_t)dk * dv * 4, kb = (size_t)C * dk * 4, vb = (size_t)C * dv * 4;
+    const size_t wb = jtk_gdn2_prefill_ws_bytes(1, C, C, dk);
     stage_t st[9] = {{S, sb, NULL}, {Q, kb, NULL}, {K, kb, NULL},   {B, kb, NULL},
                      {A, kb, NULL}, {V, vb, NULL}, {W, vb, NULL},   {NULL, vb, NULL},
-                     {NULL, jtk_gdn2_prefill_ws_bytes(1, C, C, dk), NULL}};
+                     {NULL, wb, NULL}};
     int rc = stage_in(rt, st, 9, JT_SLOT_A);
     if (rc != JT_OK) return rc;
     if (jtk_gdn2_prefill(st[0].dev, st[7].dev, st[1].dev, st[2].dev, st[5].dev, st[3].dev,
-                         st[6].dev, st[4].dev, 0, 0, 1, C, C, dk, dv, st[8].dev, jt_rt_errw(rt, rt->stream),
-                         rt->stream) != 0)
+                         st[6].dev, st[4].dev, 0, 0, 1, C, C, dk, dv, st[8].dev, wb,
+                         jt_rt_errw(rt, rt->stream), rt->stream) != 0)
         return jt_rt_err(hipErrorLaunchFailure);
     uint32_t f = 0;
     if ((rc = jt_rt_flags(rt, rt->stream, &f)) != JT_OK) return rc;
@@ -207,12 +208,13 @@ int jt_hip_gdn2_prefill(float *dS, float *dOut, const float *dQ, const float *dK
         FAIL(JT_ERR_INVAL, EINVAL);
     if (!dims_ok(dk, dv) || (C != 16 && C != 32) || T <= 0 || T % C) FAIL(JT_ERR_INVAL, EINVAL);
     if ((int64_t)T * (dk > dv ? dk : dv) > INT32_MAX) FAIL(JT_ERR_INVAL, EINVAL);
-    if (ws_bytes < jtk_gdn2_prefill_ws_bytes(H, T, C, dk) || ((uintptr_t)d_ws & 15u))
+    if (ws_bytes < jtk_gdn2_prefill_ws_min(H, T, C, dk) || ((uintptr_t)d_ws & 15u))
         FAIL(JT_ERR_INVAL, EINVAL);
     jt_rt *rt = jt_rt_get();
     if (!rt) return JT_ERR_IO;
     return jtk_gdn2_prefill(dS, dOut, dQ, dK, dV, dB, dW, dA, (int64_t)T * dk, (int64_t)T * dv,
-                            H, T, C, dk, dv, (float *)d_ws, jt_rt_errw(rt, (hipStream_t)stream), (hipStream_t)stream)
+                            H, T, C, dk, dv, (float *)d_ws, ws_bytes,
+                            jt_rt_errw(rt, (hipStream_t)stream), (hipStream_t)stream)
                ? jt_rt_err(hipErrorLaunchFailure)
                : JT_OK;
 }

@@ -24,7 +24,9 @@
 //                       launch: B, the forward substitution, Out and the
 //                       state update (:614-680, 716-842).
 //  k_gdn2_check, k_gdn2_prep_wide, k_gdn2_cols: the same where a chunk's
-//                       rows do not fit in LDS (C * dk > 4096).
+//                       rows do not fit in LDS (C * dk > 4096) or the
+//                       workspace holds no chunk's records for the scan; the
+//                       check also before a prefill in parts.
 #include "jt_dev.h"
 #include "gemm_w8a8.h"
 #include "jt_launch.h"
@@ -227,11 +229,9 @@ struct ScanRec {
 __host__ __device__ constexpr int64_t wide_rec_floats(int C, int dk) {
     return 7LL * C * dk + 2LL * C * C;
 }
-__host__ __device__ constexpr int64_t chunk_rec_floats(int C, int dk) {
+__host__ __device__ constexpr int64_t scan_rec_floats(int C, int dk) {
     const int nv = scan_blocks(dk);
-    const int64_t scan = C == 32 ? ScanRec<32>::floats(nv) : ScanRec<16>::floats(nv);
-    const int64_t wide = wide_rec_floats(C, dk);
-    return (int64_t)C * dk <= CHUNK_LDS && scan > wide ? scan : wide;
+    return C == 32 ? ScanRec<32>::floats(nv) : ScanRec<16>::floats(nv);
 }
 
 // Everything of a chunk that does not depend on the state, and the check of
@@ -548,7 +548,7 @@ template <int C, int NV, int NSUB>
 __global__ __launch_bounds__(scan_threads(C, NSUB)) void k_gdn2_scan(
     float *__restrict__ S, float *__restrict__ Out, const float *__restrict__ V,
     const float *__restrict__ W, int64_t hv, int nch, int dk, int dv,
-    const float *__restrict__ rec) {
+    const float *__restrict__ rec, const int *__restrict__ flag) {
     typedef ScanRec<C> RL;
     constexpr int R = RL::R, HB = C / 16;       // phase 1 waves, solver waves
     constexpr int OWN = R + 2 - HB;             // waves that hold state rows
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(scan_threads(C, NSUB)) void k_gdn2_scan(
     float *eb = sm + 2 * recf + sub * CGF + 4 * SK + jr * EK, *xb = eb + 4 * EK;
     const int h = blockIdx.x;
     const float *rh = rec + (int64_t)h * nch * recf;
-    bool bad = false;
+    bool bad = flag && flag[h];
     for (int c = tid; c < nch; c += NT) bad |= rh[(int64_t)c * recf + RL::flag(NV)] != 0.0f;
     if (__syncthreads_or(bad)) return;  // a rejected head keeps its S and Out
     const int j = (blockIdx.y * NSUB + sub) * 4 + jr;  // the lane's column
@@ -973,9 +973,18 @@ __global__ __launch_bounds__(256) void k_gdn2_cols(float *__restrict__ S, float 
 
 // Workspace of jtk_gdn2_prefill: H flag words (padded to 64 floats) and one
 // record per (head, chunk).
-extern "C" size_t jtk_gdn2_prefill_ws_bytes(int H, int T, int C, int dk) {
+static size_t prefill_ws(int H, int T, int C, int64_t rec_floats) {
     const int64_t flags = ((int64_t)H + 63) / 64 * 64;
-    return (size_t)(flags + (int64_t)H * (T / C) * chunk_rec_floats(C, dk)) * sizeof(float);
+    return (size_t)(flags + (int64_t)H * (T / C) * rec_floats) * sizeof(float);
+}
+extern "C" size_t jtk_gdn2_prefill_ws_min(int H, int T, int C, int dk) {
+    return prefill_ws(H, T, C, wide_rec_floats(C, dk));
+}
+// The scan's padded record is the larger one up to dk = 22 (C = 16) and 13
+// (C = 32).
+extern "C" size_t jtk_gdn2_prefill_ws_bytes(int H, int T, int C, int dk) {
+    const int64_t wide = wide_rec_floats(C, dk), scan = scan_rec_floats(C, dk);
+    return prefill_ws(H, T, C, (int64_t)C * dk <= CHUNK_LDS && scan > wide ? scan : wide);
 }
 
 // H heads, one decode step each. dk, dv in 1..1024.
@@ -1016,7 +1025,8 @@ static hipError_t launch_prep(const float *Q, const float *K, const float *B, co
 
 template <int C, int NV, int NSUB>
 static hipError_t launch_scan(float *S, float *Out, const float *V, const float *W, int64_t hv,
-                              int H, int nch, int dk, int dv, const float *rec, hipStream_t s) {
+                              int H, int nch, int dk, int dv, const float *rec, const int *flag,
+                              hipStream_t s) {
     typedef ScanRec<C> RL;
     auto kern = k_gdn2_scan<C, NV, NSUB>;
     constexpr int lds =
@@ -1035,7 +1045,8 @@ static hipError_t launch_scan(float *S, float *Out, const float *V, const float 
     }
     const int cols = 4 * NSUB;
     hipLaunchKernelGGL(kern, dim3((unsigned)H, (unsigned)((dv + cols - 1) / cols)),
-                       dim3(scan_threads(C, NSUB)), lds, s, S, Out, V, W, hv, nch, dk, dv, rec);
+                       dim3(scan_threads(C, NSUB)), lds, s, S, Out, V, W, hv, nch, dk, dv, rec,
+                       flag);
     return hipGetLastError();
 }
 
@@ -1047,24 +1058,24 @@ static hipError_t launch_scan(float *S, float *Out, const float *V, const float 
 template <int C, int NV>
 static hipError_t launch_scan_nv(float *S, float *Out, const float *V, const float *W,
                                  int64_t hv, int H, int nch, int dk, int dv, const float *rec,
-                                 hipStream_t s) {
+                                 const int *flag, hipStream_t s) {
     return (int64_t)H * ((dv + 3) / 4) <= 256
-               ? launch_scan<C, NV, 1>(S, Out, V, W, hv, H, nch, dk, dv, rec, s)
-               : launch_scan<C, NV, 2>(S, Out, V, W, hv, H, nch, dk, dv, rec, s);
+               ? launch_scan<C, NV, 1>(S, Out, V, W, hv, H, nch, dk, dv, rec, flag, s)
+               : launch_scan<C, NV, 2>(S, Out, V, W, hv, H, nch, dk, dv, rec, flag, s);
 }
 template <int C>
 static hipError_t launch_scan_c(float *S, float *Out, const float *V, const float *W,
                                 int64_t hv, int H, int nch, int dk, int dv, const float *rec,
-                                hipStream_t s) {
+                                const int *flag, hipStream_t s) {
     switch (scan_blocks(dk)) {
-        case 2: return launch_scan_nv<C, 2>(S, Out, V, W, hv, H, nch, dk, dv, rec, s);
-        case 4: return launch_scan_nv<C, 4>(S, Out, V, W, hv, H, nch, dk, dv, rec, s);
-        case 6: return launch_scan_nv<C, 6>(S, Out, V, W, hv, H, nch, dk, dv, rec, s);
-        case 8: return launch_scan_nv<C, 8>(S, Out, V, W, hv, H, nch, dk, dv, rec, s);
+        case 2: return launch_scan_nv<C, 2>(S, Out, V, W, hv, H, nch, dk, dv, rec, flag, s);
+        case 4: return launch_scan_nv<C, 4>(S, Out, V, W, hv, H, nch, dk, dv, rec, flag, s);
+        case 6: return launch_scan_nv<C, 6>(S, Out, V, W, hv, H, nch, dk, dv, rec, flag, s);
+        case 8: return launch_scan_nv<C, 8>(S, Out, V, W, hv, H, nch, dk, dv, rec, flag, s);
         default: break;
     }
     if constexpr (C == 16)
-        return launch_scan_nv<C, 16>(S, Out, V, W, hv, H, nch, dk, dv, rec, s);
+        return launch_scan_nv<C, 16>(S, Out, V, W, hv, H, nch, dk, dv, rec, flag, s);
     else
         return hipErrorInvalidValue;  // not reached: C * dk <= CHUNK_LDS
 }
@@ -1074,31 +1085,55 @@ static hipError_t launch_scan_c(float *S, float *Out, const float *V, const floa
 // head's T tokens are checked first (a head with a bad value keeps its S
 // and Out), every chunk's state-independent part is prepared in one
 // launch, then one launch runs the chunks' state updates in order. ws of
-// jtk_gdn2_prefill_ws_bytes(H, T, C, dk).
+// at least jtk_gdn2_prefill_ws_min(H, T, C, dk) bytes; where it does not hold
+// the scan's records of every chunk the sequence goes in parts of the chunks
+// that fit, after a check of all of it (8 heads x 4096 tokens, dk 8, dv 16:
+// 215 us in three parts, 194 in one), and with room for no chunk of every head
+// the kernels for larger dk take the call. The bits are the same.
 extern "C" int jtk_gdn2_prefill(float *S, float *Out, const float *Q, const float *K,
                                 const float *V, const float *B, const float *W,
                                 const float *A, int64_t hk, int64_t hv, int H, int T, int C,
-                                int dk, int dv, float *ws, uint32_t *err, hipStream_t s) {
+                                int dk, int dv, float *ws, size_t ws_bytes, uint32_t *err,
+                                hipStream_t s) {
     if (H <= 0 || H > 65535 || (C != 16 && C != 32) || T <= 0 || T % C || dk <= 0 || dv <= 0 ||
-        dk > 1024 || dv > 1024 || (int64_t)T * (dk > dv ? dk : dv) > INT32_MAX)
+        dk > 1024 || dv > 1024 || (int64_t)T * (dk > dv ? dk : dv) > INT32_MAX ||
+        ws_bytes < jtk_gdn2_prefill_ws_min(H, T, C, dk))
         return (int)hipErrorInvalidValue;
     const int nch = T / C;
-    float *rec = ws + ((int64_t)H + 63) / 64 * 64;
-    if ((int64_t)C * dk <= CHUNK_LDS) {
-        hipError_t e = C == 32
-            ? launch_prep<32>(Q, K, B, A, V, W, hk, hv, H, nch, dk, dv, rec, err, s)
-            : launch_prep<16>(Q, K, B, A, V, W, hk, hv, H, nch, dk, dv, rec, err, s);
-        if (e != hipSuccess) return (int)e;
-        e = C == 32 ? launch_scan_c<32>(S, Out, V, W, hv, H, nch, dk, dv, rec, s)
-                    : launch_scan_c<16>(S, Out, V, W, hv, H, nch, dk, dv, rec, s);
-        return (int)e;
-    }
+    const int64_t flags = ((int64_t)H + 63) / 64 * 64;
+    float *rec = ws + flags;
     int *flag = (int *)ws;
-    int le = jtk_zero_u32((uint32_t *)flag, H, s);
-    const int64_t most = (int64_t)T * (dk > dv ? dk : dv);
-    const unsigned nb = (unsigned)((most + 255) / 256 < 64 ? (most + 255) / 256 : 64);
-    hipLaunchKernelGGL(k_gdn2_check, dim3(nb, (unsigned)H), dim3(256), 0, s, Q, K, B, A, V, W,
-                       hk, hv, T * dk, T * dv, flag, err);
+    // chunks of every head whose scan records fit
+    const int64_t fit = ((int64_t)(ws_bytes / sizeof(float)) - flags) / (H * scan_rec_floats(C, dk));
+    const bool scan = (int64_t)C * dk <= CHUNK_LDS && fit > 0;
+    int le = 0;
+    if (!scan || fit < nch) {  // (in one part the preparation checks, and the scan asks its records)
+        le |= jtk_zero_u32((uint32_t *)flag, H, s);
+        const int64_t most = (int64_t)T * (dk > dv ? dk : dv);
+        const unsigned nb = (unsigned)((most + 255) / 256 < 64 ? (most + 255) / 256 : 64);
+        hipLaunchKernelGGL(k_gdn2_check, dim3(nb, (unsigned)H), dim3(256), 0, s, Q, K, B, A, V,
+                           W, hk, hv, T * dk, T * dv, flag, err);
+    }
+    if (scan) {
+        const int part = (int)(fit < nch ? fit : nch);
+        const int *whole = part < nch ? flag : nullptr;
+        for (int c0 = 0; c0 < nch; c0 += part) {
+            const int m = part < nch - c0 ? part : nch - c0;
+            const int64_t k0 = (int64_t)c0 * C * dk, v0 = (int64_t)c0 * C * dv;
+            hipError_t e = C == 32
+                ? launch_prep<32>(Q + k0, K + k0, B + k0, A + k0, V + v0, W + v0, hk, hv, H, m,
+                                  dk, dv, rec, err, s)
+                : launch_prep<16>(Q + k0, K + k0, B + k0, A + k0, V + v0, W + v0, hk, hv, H, m,
+                                  dk, dv, rec, err, s);
+            if (e != hipSuccess) return (int)e;
+            e = C == 32 ? launch_scan_c<32>(S, Out + v0, V + v0, W + v0, hv, H, m, dk, dv, rec,
+                                            whole, s)
+                        : launch_scan_c<16>(S, Out + v0, V + v0, W + v0, hv, H, m, dk, dv, rec,
+                                            whole, s);
+            if (e != hipSuccess) return (int)e;
+        }
+        return le;
+    }
     hipLaunchKernelGGL(k_gdn2_prep_wide, dim3((unsigned)nch, (unsigned)H), dim3(256), 0, s, Q,
                        K, B, A, hk, C, dk, flag, rec);
     auto cols = C == 32 ? k_gdn2_cols<32> : k_gdn2_cols<16>;

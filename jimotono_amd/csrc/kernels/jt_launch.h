@@ -322,13 +322,15 @@ int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, int k, int S
 int jtk_gdn2_decode(float *S, float *O, const float *q, const float *k, const float *v,
                     const float *b, const float *w, const float *alpha, int H, int dk, int dv,
                     uint32_t *err, hipStream_t s);
+/* the workspace for the fastest kernels, and the least that is taken */
 size_t jtk_gdn2_prefill_ws_bytes(int H, int T, int C, int dk);
+size_t jtk_gdn2_prefill_ws_min(int H, int T, int C, int dk);
 /* T tokens per head (T % C == 0) in T/C chunks; a head with a bad input
  * value anywhere keeps its S and Out (EF_NONFINITE_INPUT). */
 int jtk_gdn2_prefill(float *S, float *Out, const float *Q, const float *K, const float *V,
                      const float *B, const float *W, const float *A, int64_t hk, int64_t hv,
-                     int H, int T, int C, int dk, int dv, float *ws, uint32_t *err,
-                     hipStream_t s);
+                     int H, int T, int C, int dk, int dv, float *ws, size_t ws_bytes,
+                     uint32_t *err, hipStream_t s);
 int jtk_gdn2_l2norm(const float *x, float *y, int rows, int n, float eps, hipStream_t s);
 
 #ifdef __cplusplus

@@ -121,6 +121,31 @@ def test_validation_before_device_work(lib):
     assert bf(1, C.byref(b)) == 0 and b.value == 4
 
 
+@pytest.mark.parametrize("C_,dk", [(16, 1), (16, 22), (16, 23), (32, 1), (32, 13), (32, 14),
+                                   (32, 128), (16, 257)])
+def test_gdn2_prefill_takes_the_documented_workspace(lib, C_, dk):
+    """jt_hip_gdn2_prefill takes a workspace of the size that hip_gdn2.h
+    states, 4*ceil(H/64)*64 + H*(T/C)*(7*C*dk + 2*C*C)*4 bytes, and refuses a
+    smaller one; the size function never asks for less. (Without a GPU an
+    accepted call ends with JT_ERR_IO, before any device work.)"""
+    try:
+        import torch
+        if torch.cuda.is_available():
+            pytest.skip("a GPU is visible")
+    except ImportError:
+        pass
+    H, T, dv = 3, 2 * C_, 8
+    need = 4 * 64 + H * 2 * (7 * C_ * dk + 2 * C_ * C_) * 4
+    size = lib.jt_hip_gdn2_prefill_ws_bytes
+    size.restype = C.c_size_t
+    assert size(H, T, C_, dk) >= need
+    f = lib.jt_hip_gdn2_prefill
+    f.argtypes = [C.c_void_p] * 8 + [C.c_int] * 5 + [C.c_void_p, C.c_size_t, C.c_void_p]
+    for nb, rc, en in ((need, 3, E.ENODEV), (need - 1, 2, E.EINVAL)):
+        C.set_errno(0)
+        assert f(*[64] * 8, H, T, C_, dk, dv, 64, nb, None) == rc and C.get_errno() == en
+
+
 def test_api_refuses_without_library(monkeypatch, tmp_path):
     import jimotono_amd.api as api
     monkeypatch.setattr(api, "LIB_PATH", str(tmp_path / "missing.so"))

@@ -308,6 +308,44 @@ def test_gdn2_prefill_device_row_blocks(jt, orc, torch_cuda, H, T, C_, dk, dv):
         assert same(S1[h], Sh), h
 
 
+@pytest.mark.parametrize("C_,dk,nch", [(16, 1, 3), (16, 1, 7), (16, 22, 3), (32, 5, 3),
+                                       (32, 13, 1), (32, 13, 5)])
+def test_gdn2_prefill_device_smallest_workspace(jt, orc, torch_cuda, C_, dk, nch):
+    """A workspace of the documented least size where the fast kernels'
+    records are larger: the sequence in parts (of 1, 2, 1 and 4 chunks), or
+    the kernels for larger dk where no chunk of every head fits; the same
+    bits (against the oracle's chunk chain), and a head with a bad value in
+    the last chunk kept as it was from the first part on."""
+    torch = torch_cuda
+    announce(f"jt_hip_gdn2_prefill smallest workspace C={C_} dk={dk} chunks={nch}")
+    H, T, dv = 3, nch * C_, 9
+    rng = np.random.default_rng(C_ + dk)
+    S = (rng.standard_normal((H, dk, dv)) * 0.3).astype(np.float32)
+    Q, K, B = (rng.standard_normal((H, T, dk)).astype(np.float32) for _ in range(3))
+    A = rng.uniform(0.5, 1, (H, T, dk)).astype(np.float32)
+    V, W = (rng.standard_normal((H, T, dv)).astype(np.float32) for _ in range(2))
+    V[1, T - 1, 2] = np.inf
+    nb = 4 * 64 + H * nch * (7 * C_ * dk + 2 * C_ * C_) * 4
+    assert jt.lib().jt_hip_gdn2_prefill_ws_bytes(H, T, C_, dk) > nb
+    ws = torch.empty(nb, dtype=torch.uint8, device="cuda")
+    dS, dOut = _t(torch, S), torch.full((H, T, dv), 42.0, device="cuda")
+    ins = [_t(torch, x) for x in (Q, K, V, B, W, A)]
+    rc = jt.lib().jt_hip_gdn2_prefill(*[t.data_ptr() for t in (dS, dOut, *ins)], H, T, C_, dk,
+                                      dv, ws.data_ptr(), nb, None)
+    assert rc == 0
+    assert jt.sync_errors() & jt.EF_NONFINITE_INPUT
+    S1, O1 = dS.cpu().numpy(), dOut.cpu().numpy()
+    assert same(S1[1], S[1]) and (O1[1] == 42.0).all()
+    for h in (0, 2):
+        Sh = S[h]
+        for c0 in range(0, T, C_):
+            sl = slice(c0, c0 + C_)
+            rc, Sh, Oh = orc.gdn2_prefill_chunk(Sh, Q[h, sl], K[h, sl], V[h, sl], B[h, sl],
+                                                W[h, sl], A[h, sl])
+            assert rc == 0 and same(O1[h, sl], Oh), (h, c0)
+        assert same(S1[h], Sh), h
+
+
 def test_gdn2_prefill_full_size(jt, orc, torch_cuda):
     """The prefill benchmark's shape: 8 heads x 4096 tokens of 128x128
     states in chunks of 32, every head's state and every output against the
