@@ -104,14 +104,14 @@ def test_bwd_vs_oracle(jt, orc, case):
 
 
 @pytest.mark.parametrize("case", [
-    (300, 136, 130, 520, 2, 1, 21, None),   # matrix-core form in all three products
-    (70, 260, 68, 530, 3, 0, 22, 1.0),      # no shared experts, one column tile of 68
+    (300, 136, 130, 520, 2, 1, 21, None),   # matrix-core row products, 2 x 4 weight gradients
+    (70, 260, 68, 530, 3, 0, 22, 1.0),      # no shared experts, one row an expert
     (130, 48, 40, 12, 2, 1, 23, None)])     # the smallest tiles, K = 130 of the shared expert
 def test_bwd_tile_forms_vs_oracle(jt, orc, case):
     """The product forms at ragged tiles: 64 x 128 with products from the
     matrix cores (1024 tiles and more), 4 x 2, 2 x 4 and 2 x 2 outputs a
     thread below. Every form keeps the order and the two roundings, so the
-    bounds are check()'s."""
+    bounds are check()'s. (The matrix-core weight gradients: the test below.)"""
     announce(f"moe_bwd_batch tile forms {case}")
     c = bwd_case(*case)
     want = orc.moe_bwd_batch(*bwd_args(c))
@@ -119,6 +119,46 @@ def test_bwd_tile_forms_vs_oracle(jt, orc, case):
     o = jt.moe_bwd_batch(*bwd_args(c))
     assert o["rc"] == 0
     check(o, want, label=str(case))
+
+
+@pytest.mark.parametrize("case,tiny", [
+    # matrix-core weight gradients, K = 130 and about 52; no shared expert
+    ((130, 650, 200, 20, 8, 1, 25, None), False), ((130, 644, 200, 20, 8, 0, 26, None), False),
+    ((40, 641, 129, 20, 10, 1, 27, None), True),   # K = 40 and about 20
+    # matrix-core row products
+    ((300, 136, 130, 520, 2, 1, 21, None), False), ((300, 136, 130, 520, 2, 1, 21, None), True),
+    # sums in registers throughout
+    ((130, 48, 40, 12, 2, 1, 23, None), False), ((130, 48, 40, 12, 2, 1, 23, None), True)])
+def test_bwd_products_to_the_bit(jt, orc, case, tiny):
+    """With every gate value 0 or above 38 the sigmoid is exactly 1/2 or 1
+    (exp(-38) < 2^-54), so no output depends on the rounding of exp and all of
+    them must equal the oracle's to the bit: per product one rounded multiply
+    and one rounded add, k ascending. `tiny`: most products of the row GEMMs
+    and of dWg are subnormal, as are most of the rows that the later products
+    read (Wgate = 0: the gate path's terms in dX would be 1e20 times larger)."""
+    announce(f"moe_bwd_batch products to the bit {case} tiny={tiny}")
+    c = bwd_case(*case)
+    rng = np.random.default_rng(case[6])
+    for g in ("Gsel", "Gs"):
+        if c[g] is not None:
+            c[g] = np.where(rng.random(c[g].shape) < 0.5, 0, 38 + np.abs(c[g])).astype(np.float32)
+    if tiny:
+        for x in ("dY", "Wd", "Wd_s"):
+            if c[x] is not None:
+                c[x] = (c[x] * np.float32(1e-20)).astype(np.float32)
+        c["Wgate"] = np.zeros_like(c["Wgate"])
+    want = orc.moe_bwd_batch(*bwd_args(c))
+    assert want["rc"] == 0
+    if tiny:
+        for nm in ("dWg", "dX"):
+            a = np.abs(want[nm])
+            assert ((a > 0) & (a < np.finfo(np.float32).tiny)).mean() > 0.5, nm
+    o = jt.moe_bwd_batch(*bwd_args(c))
+    assert o["rc"] == 0
+    for nm in OUTS:
+        if nm in want:
+            a, b = bits(o[nm]), bits(want[nm])
+            assert np.array_equal(a, b), (nm, int((a != b).sum()), a.size)
 
 
 def test_bwd_without_logits(jt, orc):

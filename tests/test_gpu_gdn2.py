@@ -236,14 +236,14 @@ def test_gdn2_prefill_device_heads(jt, orc, torch_cuda):
         assert same(S1[h], Sh), h
 
 
-@pytest.mark.parametrize("H,T,C_,dk,dv", [(3, 64, 16, 64, 48),     # 16-row chunks, 8-column blocks
-                                          (4, 48, 16, 32, 1024),   # 16-row chunks, 16-column blocks
+@pytest.mark.parametrize("H,T,C_,dk,dv", [(3, 64, 16, 64, 48),     # 16-row chunks, 4-column blocks
+                                          (4, 48, 16, 32, 1024),   # 16-row chunks, 8-column blocks
                                           (2, 64, 32, 32, 1024)])  # 32-row chunks, 8-column blocks
 def test_gdn2_prefill_device_block_widths(jt, orc, torch_cuda, H, T, C_, dk, dv):
-    """Every column-block width of the prefill's state kernel: blocks of
-    128/C columns while the grid has fewer than 256 blocks of 256/C, then
-    the wide blocks (4 heads x 1024 columns at C=16, 2 x 1024 at C=32),
-    each head's state and outputs against the oracle's chunk chain."""
+    """Both column-block widths of the prefill's state kernel: one group of 4
+    columns a block up to 256 groups, two above (4 heads x 1024 columns at
+    C=16, 2 x 1024 at C=32), each head's state and outputs against the
+    oracle's chunk chain."""
     torch = torch_cuda
     announce(f"jt_hip_gdn2_prefill H={H} T={T} C={C_} {dk}x{dv}")
     rng = np.random.default_rng(H * 100 + C_ + dv)
@@ -269,13 +269,17 @@ def test_gdn2_prefill_device_block_widths(jt, orc, torch_cuda, H, T, C_, dk, dv)
 
 @pytest.mark.parametrize("H,T,C_,dk,dv", [
     (1, 16, 16, 1, 5),      # one chunk, one value, a partial column group
-    (2, 64, 32, 31, 3), (1, 96, 32, 33, 259),   # around 2 blocks of 16 rows; two groups a block
-    (2, 64, 32, 97, 10), (1, 64, 32, 127, 7),   # 6 and 8 blocks with padded rows
+    (2, 64, 32, 31, 3), (1, 96, 32, 33, 259),   # around 2 blocks of 16 rows; 65 column groups
+    (2, 64, 32, 97, 10), (1, 64, 32, 127, 7),   # 8 blocks with padded rows
     (2, 48, 16, 64, 6), (1, 48, 16, 90, 1023),  # 4 and 6 blocks, C = 16
-    (1, 32, 16, 129, 9), (2, 48, 16, 250, 530)])  # 16 blocks
+    (1, 32, 16, 129, 9), (2, 48, 16, 250, 530),  # 16 blocks
+    # two groups a block (above 256), an odd number of them a head: the second
+    # group of the last block holds no column
+    (2, 96, 32, 64, 521), (2, 96, 32, 96, 521), (2, 96, 32, 128, 521),
+    (2, 48, 16, 64, 521), (2, 48, 16, 96, 521), (2, 48, 16, 128, 521)])
 def test_gdn2_prefill_device_row_blocks(jt, orc, torch_cuda, H, T, C_, dk, dv):
-    """Every row-block count of the state kernel at its edges, with ragged
-    columns, zero-norm rows, signed zeros and alphas of 0 and 1: bit for bit
+    """Every row-block count of the state kernel at its edges, with one and two
+    column groups a block, ragged columns, zero-norm rows, signed zeros and alphas of 0 and 1: bit for bit
     the oracle's chunk chain (the tolerance is none: every chain keeps the
     reference's order and roundings)."""
     torch = torch_cuda
