@@ -762,14 +762,22 @@ static int moe_forward(jt_hip_moe *L, const float *dX, const int32_t *d_ids,
      * the codes, 0.332-0.334 forking after the approximate logits) */
     const int fork_late = fork && fast;
     if (fork && !fork_late) le |= fork_shared(L, T, fused, err, s);
-    /* 16-row tiles when experts average at most 16 rows and either the
-     * one-launch FFN of such tiles takes the shape or the tiles are few: the
-     * generic 16-row kernel costs about 0.6 us a tile (512 experts, n 2048,
-     * h 512, one shared expert: 8 tokens 72 us against 83 with 64-row tiles, 16
-     * tokens 122 against 119, 64 tokens 224 against 181, 1024 tokens 585
-     * against 337) */
+    /* 16-row tiles when experts average at most 16 rows and the one-launch FFN
+     * of such tiles takes the shape. The generic 16-row kernels cost about
+     * 0.6 us a tile (n 2048, h 512) and a launch more, the 64-row ones 50-110 us
+     * however few tiles there are, so what is faster depends on how many
+     * experts the pairs fall on, which the host does not know: 64-row tiles
+     * from 4096 pairs on, 256 tiles of 16 rows even if all fall on topk
+     * experts. Of h = 256 and 512 a gate/up tile is one block, which needs the
+     * longer rows to pay (16-row / 64-row us of a caller-routed call, top-8,
+     * even / Zipf(1.1) / the same 8 experts; 512 experts, n 2048, h 512: 4096
+     * pairs 335 / 360 / 152 against 169 / 242 / 113, 2048 pairs 319 / 260 / 95
+     * against 161 / 171 / 109, 192 pairs 85 / 68 / 30 against 66 / 73 / 52; 256
+     * experts, n 1024, h 512, 4096 pairs: 97 / 104 / 77 against 72 / 124 / 82;
+     * n 1536, h 256, 4096 pairs: 101 / 108 / 80 against 66 / 103 / 75). */
     const int ffn16 = h == 256 && n % 256 == 0 && n <= 1024;
-    const int R = Tk <= 16 * E && (ffn16 || (Tk < E ? Tk : E) < 128) ? 16 : 64;
+    const int tall = !ffn16 && Tk >= 4096 && (n >= 1536 || (h != 256 && h != 512));
+    const int R = Tk <= 16 * E && !tall ? 16 : 64;
     /* tiles: at most Tk / R plus one per expert that holds a pair */
     const int max_tiles = Tk / R + (E < Tk ? E : Tk);
     /* Decode with the shared experts concatenated: top-k, the pair sort and

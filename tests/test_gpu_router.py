@@ -182,14 +182,15 @@ def test_router_logits_any_width(jt, orc, T, n, E):
 
 
 def test_routed_tile_height_same_rows(jt, torch_cuda):
-    """Experts of 512 hidden rows take 64-row tiles from 128 tiles on and
-    16-row ones below: a token's output does not depend on it."""
+    """At n = 1536 the routed experts take 64-row tiles from 4096 pairs on,
+    also where they average 16 rows, and 16-row ones below: a token's output
+    does not depend on it."""
     torch = torch_cuda
     announce("routed tile heights")
-    n, h, E, k, T = 256, 512, 160, 8, 40
+    n, h, E, k, T = 1536, 512, 256, 8, 512
     g = torch.Generator(device="cuda").manual_seed(5)
     rn = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
-    L = jt.MoE(n, h, E, k, 0, 0, T, rn(E, n), rn(E, h, n) / 16, rn(E, h, n) / 16,
+    L = jt.MoE(n, h, E, k, 0, 0, T, rn(E, n), rn(E, h, n) / 39, rn(E, h, n) / 39,
                rn(E, h, n) / 22)
     X = rn(T, n)
     Y, Y8 = torch.empty_like(X), torch.empty(8, n, device="cuda")
