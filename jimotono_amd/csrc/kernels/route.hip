@@ -250,9 +250,10 @@ __global__ __launch_bounds__(256) void k_router_logits_tile(const float *__restr
 extern "C" int jtk_router_logits(const float *X, const float *Wg, int T, int E, int n,
                                  float *logits, uint32_t *err, hipStream_t s) {
     const int64_t tiles = (int64_t)((T + 15) / 16) * ((E + 15) / 16);
-    // (512 experts, n 2048: 256 tokens, 512 tiles: the layer 410 us against 463
-    // with 64 x 64 tiles; 1024 tokens: 732 against 607)
-    if (tiles < 1024) {
+    // up to three blocks a CU (a layer of 300 small experts, n 2048, with 16 x 16
+    // and with 64 x 64 tiles: 700 tiles 149 and 156 us, 850 tiles 182 and 157,
+    // 2048 tiles 345 and 167; n 256: 700 tiles 53.7 and 54.3, 850 tiles 61 and 55)
+    if (tiles <= 768) {
         hipLaunchKernelGGL(k_router_logits_tile, dim3((unsigned)tiles), dim3(256), 0, s, X, Wg, T,
                            E, n, logits, err);
     } else {
