@@ -24,6 +24,8 @@
 //  EPI_STORE (D^T X weight gradients).
 //  k_bwd_dx     : dX = (float)(gate + routed rows in perm order + shared)
 //                 in fp64 (:2236-2245, 2354-2363, 2411-2429)
+#include <algorithm>
+
 #include "jt_dev.h"
 #include "jt_launch.h"
 
@@ -347,32 +349,46 @@ __global__ __launch_bounds__(256, EPI == EPI_DUAL ? 2 : 3) void k_bwd_gemm_mx(Ge
 }
 
 // rows: row tiles of 64 (MODE_ROWS, both sides) or output rows
-// (MODE_WGRAD); groups: grid z; many: no serial sum is long beside the whole
-// launch. The matrix-core form from 1024 tiles of 64 x 128 on, where it has
-// two waves or more on a SIMD (4096 tokens, n 1024, h 256, 64 experts top-8
-// and one shared: 481, 900 and 1164 us against 541, 977 and 1237 with 4 x 4
-// outputs a thread); a step of its sum takes 400 cycles, so a shared expert's
-// K = T must not outlast the rest (`many`; n 512, h 256, 32 experts top-4 and
-// one shared at T = 4096: 687 us against 469 with 2 x 4). Below that a block's
-// time is its serial K loop and small tiles are faster (64 tokens of the first
-// layer, 146 and 584 tiles: 104 and 147 us with 4 x 2 outputs a thread, 137
-// and 151 with 4 x 4, 162 and 168 in the matrix-core form; 27 tiles of weight
-// gradients with K = 512: 30 us with 2 x 2, 47 with 2 x 4, 63 with 4 x 4).
+// (MODE_WGRAD); groups: grid z; blocks: blocks of 64 x 64 outputs that have
+// work, if the pairs spread evenly over the experts; serial, mx: MODE_WGRAD,
+// see below. A form with 4x4 outputs a thread, or
+//  - the matrix-core one (64 x 128 tiles, two blocks a CU with two sums, else
+//    three) where the tiles hold little padding, are more than one round of
+//    blocks and fill three quarters of the rounds: two sums, 900 to 1024 tiles 1
+//    to 3.6% of the call below 4x4, 1056 to 1152 2 to 3% above; SwiGLU, 832 to
+//    1024 tiles 1 to 1.6% above, from 1216 on 0.2 to 1.6% below. (One round of two
+//    sums took 6% less or 7% more: where the list's unused blocks fall decides
+//    it.) With h = 64, half of a tile padding, 7.5% above (16384 tokens, 64
+//    experts top-8).
+//  - 4x2 (row GEMMs) where blocks are few and a block's serial K loop is the
+//    time: up to 544 blocks with two sums (448: 7 to 9% below 4x4, 528 and 544: 2%
+//    above to 6% below, 768: 4% above) and 768 of the SwiGLU product (448: 6.5%
+//    below, 704 and 768: 3.2% below to 2.4% above).
+// (The calls: 64 to 4096 tokens, 16 to 128 experts, n 256 to 2048, h 64 to 512.)
 template <bool AT, bool BT, int EPI, int MODE>
-int launch_gemm(const GemmP &p, unsigned rows, unsigned groups, bool many, hipStream_t s) {
+int launch_gemm(const GemmP &p, unsigned rows, unsigned groups, int64_t blocks, bool serial,
+                bool mx, hipStream_t s) {
     if (rows == 0 || p.N <= 0 || groups == 0) return 0;
     auto grid = [&](int BM, int BN) {
         return dim3(MODE == MODE_ROWS ? rows : (rows + BM - 1) / BM,
                     (unsigned)((p.N + BN - 1) / BN), groups);
     };
     const dim3 g = grid(64, 128);
-    const int64_t tiles = (int64_t)g.x * g.y * g.z;
-    if (tiles >= 1024 && many) {
+    const int64_t tiles = blocks / 2, slots = 256 * (EPI == EPI_DUAL ? 2 : 3);
+    const bool full = MODE == MODE_ROWS ? tiles > slots && 4 * tiles > 3 * slots *
+                                              ((tiles + slots - 1) / slots)
+                                        : mx && tiles >= 1024;
+    const bool few = MODE == MODE_ROWS ? blocks <= (EPI == EPI_DUAL ? 544 : 768)
+                                       : serial || blocks < 512;
+    if (full && 128 * (int64_t)g.y <= p.N + p.N / 8) {
         hipLaunchKernelGGL((k_bwd_gemm_mx<AT, BT, EPI, MODE>), g, dim3(256), 0, s, p);
+    } else if (!few) {
+        hipLaunchKernelGGL((k_bwd_gemm<AT, BT, EPI, MODE, 4, 4>), grid(64, 64), dim3(256), 0, s,
+                           p);
     } else if constexpr (MODE == MODE_ROWS) {
         hipLaunchKernelGGL((k_bwd_gemm<AT, BT, EPI, MODE, 4, 2>), grid(64, 32), dim3(256), 0, s,
                            p);
-    } else if (tiles >= 64) {
+    } else if (blocks >= 128) {
         hipLaunchKernelGGL((k_bwd_gemm<AT, BT, EPI, MODE, 2, 4>), grid(32, 64), dim3(256), 0, s,
                            p);
     } else {
@@ -889,6 +905,8 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
     le |= jtk_make_tiles(w->off32, E, BM_ROWS, w->tiles, w->ntiles, s);
     const unsigned mt = (unsigned)(Tk / BM_ROWS + E);  // bound on the routed tile count
     const int mt_sh = (int)cdiv(T, BM_ROWS);
+    // row tiles to expect: each expert's last one is half full on average
+    const int64_t ex = S * mt_sh + std::max(std::min(E, Tk), Tk / BM_ROWS + E / 2);
     // Dg, Du, S = SwiGLU backward of (rows Wd^T): shared experts on all
     // tokens with dY unweighted, routed experts on their perm rows
     GemmP p{};
@@ -907,7 +925,8 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
         b.G = io->Gsel, b.U = io->Usel, b.rowq = w->rowq, b.ldg = h;
         b.K = n, b.tiles = (const int4 *)w->tiles, b.ntiles = w->ntiles;
     }
-    le |= launch_gemm<false, true, EPI_DSWIGLU, MODE_ROWS>(p, p.nsh + mt, 1, true, s);
+    le |= launch_gemm<false, true, EPI_DSWIGLU, MODE_ROWS>(p, p.nsh + mt, 1, ex * cdiv(h, 64), false,
+                                                           false, s);
     // dx rows = (float)((double)(Dg Wg) + (double)(Du Wu))
     p = GemmP{};
     p.err = err, p.N = n, p.nsh = S * mt_sh, p.mt_sh = mt_sh;
@@ -923,7 +942,8 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
         b.C[0] = w->Dxe, b.ldc = n;
         b.K = h, b.tiles = (const int4 *)w->tiles, b.ntiles = w->ntiles;
     }
-    le |= launch_gemm<false, false, EPI_DUAL, MODE_ROWS>(p, p.nsh + mt, 1, true, s);
+    le |= launch_gemm<false, false, EPI_DUAL, MODE_ROWS>(p, p.nsh + mt, 1, ex * cdiv(n, 64), false,
+                                                         false, s);
     // weight gradients D^T rows: dWg = Dg^T X, dWu = Du^T X, dWd = S^T dY
     // (routed: weighted dY rows, over the expert's rows in perm order)
     p = GemmP{};
@@ -940,10 +960,19 @@ extern "C" int jtk_bwd_batch(const jtk_bwd_io *io, int T, int n, int h, int E, i
         b.C[0] = io->dWg, b.C[1] = io->dWu, b.C[2] = io->dWd, b.ldc = n, b.sCg = nh;
         b.M = h, b.koff = w->off32;
     }
-    // a tile's sum over the T tokens of a shared expert against all tiles'
-    // sums, 400 cycles a step and 0.33 ns a step of the whole chip
-    const bool many = S == 0 || 3LL * (S + k) * cdiv(h, 64) * cdiv(n, 128) >= 400;
-    le |= launch_gemm<true, false, EPI_STORE, MODE_WGRAD>(p, h, 3 * (S + E), many, s);
+    // A sum over all T tokens (a shared expert's, or one that every token
+    // chose) takes T steps of 154 ns with the matrix cores, 123 with 4x4, 92 with
+    // 2x4, 61 with 2x2; the chip does a tile's step in 0.33 ns, T * steps of them
+    // in all. The forms cross where that says (one shared expert, 4096 tokens: 240
+    // steps 2x4 83 us below 4x4 of 1119, 324 equal, 360 43 above of 1409; matrix
+    // cores 53 above 4x4 of 1670 at 432 steps, 40 below of 2006 at 540). Without a
+    // shared expert 4x4 below 540 unless blocks are few: 2x4 is 18 to 50 us above it
+    // with even routing, and if all tokens choose the same experts the matrix cores
+    // 122 to 142 above of 1150.
+    const int64_t steps = 3LL * (S + k) * cdiv(h, 64) * cdiv(n, 128);
+    le |= launch_gemm<true, false, EPI_STORE, MODE_WGRAD>(
+        p, h, 3 * (S + E), 3LL * (S + E) * cdiv(h, 64) * cdiv(n, 64), S && steps < 330,
+        steps >= 540, s);
     hipLaunchKernelGGL(k_bwd_dx, dim3((unsigned)T, cdiv(n, 1024)), dim3(256), 0, s, io->Wgate,
                        w->gate_e, w->gate_dl, w->gate_n, w->tokpos, w->tokcnt, w->Dxe, w->SDxe,
                        S, T, k, n, io->dX, err);
