@@ -193,8 +193,8 @@ __global__ __launch_bounds__(256) void k_gdn2_decode(float *__restrict__ S, floa
 // ---- prefill with a chunk's operands in LDS (C * dk <= CHUNK_LDS) ----
 //
 // Record of one (head, chunk), written by k_gdn2_prep in the order in which
-// k_gdn2_scan reads it, so that a wave copies it to LDS with linear
-// 16-byte LDS-DMA (floats; dk padded to nv = scan_blocks(dk) blocks of 16
+// k_gdn2_scan reads it, so that a wave copies it to LDS with linear 16-byte
+// loads and stores (floats; dk padded to nv = scan_blocks(dk) blocks of 16
 // with zeros, roles r < C/8: rows 16*(r % (C/16)) + tt of -ke*CF for the first
 // C/16 roles, of q*CF for the others, CF the forward decay products):
 //   P    [block][s/4][tt][s%4]        16x16 blocks (0,0), (1,0), (1,1) of P
@@ -245,7 +245,7 @@ __host__ __device__ constexpr int64_t scan_rec_floats(int C, int dk) {
 // product in a register, 16 + 16 sums in registers. The operands are held
 // transposed, [i][t] at a stride of C + 4, so that the 16 rows of an i are
 // four 16-byte LDS reads an array (48 4-byte reads an i made the walk wait
-// on LDS issue: 88 000 cycles a block against 25 000). The waves without a
+// on LDS issue). The waves without a
 // block write the decay products and the row weights meanwhile.
 template <int C>
 __global__ __launch_bounds__(256) void k_gdn2_prep(
@@ -529,8 +529,9 @@ __device__ __forceinline__ float solve16(float x, const float4 (&m)[4], int tt) 
 //   phase 3, the other waves without a solve to do: rows i = 16v + tt of the
 //            state: S <- CF S + sum_s WG[s][i] E_s.
 // The last two waves also copy the next chunk's record to LDS during phase
-// 1 (by LDS-DMA, 60 to 90 cycles of the issuing wave a KiB, it held the
-// other waves for 800 cycles a chunk or one wave for 5000).
+// 1, through registers (by LDS-DMA, 60 to 90 cycles of the issuing wave a
+// KiB, the copy held the other waves for 800 cycles a chunk or one wave for
+// 5000).
 // A step of a chain is a multiply and an add (two roundings), and its
 // operands come 4 at a time from LDS, the next 16 steps' while the current
 // ones run: a row's M, WG, L or P values and the column's S or E values

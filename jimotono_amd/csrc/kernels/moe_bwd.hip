@@ -17,8 +17,8 @@
 //                 stable expert sort of the kept pairs
 // Expert path (steps 5-6): three bit-exact fp32 GEMM forms (per output, a
 // k-ascending sequence of rounded multiplies and rounded adds, as
-// src/moe_gemm.c:47-89), k_bwd_gemm_mx on 64x128 tiles for large layers,
-// k_bwd_gemm on smaller ones:
+// src/moe_gemm.c:47-89), k_bwd_gemm_mx on 64x128 tiles where they are
+// many, else k_bwd_gemm:
 //  <AT, BT, EPI> with EPI_DSWIGLU (dY Wd^T -> SwiGLU backward
 //  -> Dg, Du, S), EPI_DUAL ((float)((double)Dg Wg + (double)Du Wu)) and
 //  EPI_STORE (D^T X weight gradients).
@@ -111,7 +111,6 @@ struct Chunk {
     }
 };
 
-// acc[i][j] += a[i] * b[j]: one rounded multiply, one rounded add
 template <int N>
 __device__ __forceinline__ void ld_row(float (&v)[N], const float *s) {
     if constexpr (N % 4 == 0) {
@@ -122,6 +121,7 @@ __device__ __forceinline__ void ld_row(float (&v)[N], const float *s) {
         for (int i = 0; i < N; i += 2) *(float2 *)&v[i] = *(const float2 *)(s + i);
     }
 }
+// acc[i][j] += a[i] * b[j]: one rounded multiply, one rounded add
 template <int TM, int TN>
 __device__ __forceinline__ void mul_add(float (&acc)[TM][TN], const float *as, const float *bs) {
     float av[TM], bv[TN];

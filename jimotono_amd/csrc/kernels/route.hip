@@ -3,10 +3,9 @@
 //  k_router_logits : logits[t][e] = (float)dot(X[t], Wgate[e]) in fp64 with
 //                    the reference's four lane partials over j % 4, combined
 //                    as (l0+l1)+(l2+l3), then the tail (src/moe_layer.c:67-86,
-//                    1118-1137), on fp64 matrix cores, beside the tokens'
-//                    codes. Products of two floats are exact in fp64, so a
-//                    fused step rounds exactly like the reference's separate
-//                    multiply and add.
+//                    1118-1137), on fp64 matrix cores. Products of two
+//                    floats are exact in fp64, so a fused step rounds exactly
+//                    like the reference's separate multiply and add.
 //  k_topk          : top-k by value with ties to the lower index, softmax
 //                    over the selected k in fp64 (src/routing.c:16-76).
 //  k_sort_*        : stable counting sort of the (token, slot) pairs by
