@@ -529,7 +529,9 @@ def calib_bench(blocks=512, iters=4000):
     from different waves of one SIMD (split) or from the same wave (same):
     overlap = (t_mfma + t_valu - t_mixed) / min(t_mfma, t_valu), 1 for
     perfect overlap and 0 when the two run one after the other. Then the
-    MFMA rate with LDS-fed operands (and a barrier per 16 MFMAs), and the
+    MFMA rate with LDS-fed operands (and a barrier per 16 MFMAs), the rates
+    of the backward's separately rounded fp32 products (v_mul and v_add, and
+    zero-accumulator MFMAs with v_add) and of the router's fp64 MFMAs, and the
     128x256 tile GEMM's rate with its operands in HBM or aliased into L2.
     512 blocks of 8 waves: 4 waves per SIMD. Times per wave iteration are in
     ns per SIMD (each SIMD runs blocks * 8 / 1024 waves)."""
@@ -538,7 +540,7 @@ def calib_bench(blocks=512, iters=4000):
     Lc.jt_calib_issue.argtypes = [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_float)]
     Lc.jt_calib_tile.argtypes = [C.c_int, C.POINTER(C.c_float), C.POINTER(C.c_double)]
     t = []
-    for mode in range(9):
+    for mode in range(12):
         ms = C.c_float()
         rc = Lc.jt_calib_issue(mode, blocks, iters, C.byref(ms))
         assert rc == 0, f"jt_calib_issue({mode}) rc={rc}"
@@ -560,8 +562,14 @@ def calib_bench(blocks=512, iters=4000):
         "overlap_fp64_same_wave": ovl(t[0], t[4], t[6]),
         "mfma_lds_fed_tops": tops(7),
         "mfma_lds_fed_barrier_tops": tops(8),
+        "fp32_mul_add_ns_per_2048": ns(9) / 2,
+        "fp32_mul_add_tproducts": 1024e-3 * 2048 / (ns(9) / 2),
+        "fp32_mfma_add_ns_per_2048": ns(10) / 2,
+        "fp32_mfma_add_tproducts": 1024e-3 * 2048 / (ns(10) / 2),
+        "mfma_f64_16x16x4_ns_each": ns(11) / 16,
         "ms": dict(zip(["mfma", "fp32", "mfma_fp32_split", "mfma_fp32_same", "fp64",
-                        "mfma_fp64_split", "mfma_fp64_same", "mfma_lds", "mfma_lds_barrier"],
+                        "mfma_fp64_split", "mfma_fp64_same", "mfma_lds", "mfma_lds_barrier",
+                        "fp32_mul_add", "fp32_mfma_add", "mfma_fp64"],
                        t)),
     }
     tile = {}
@@ -895,7 +903,8 @@ def proj_bench(np, torch, api, stream):
 BWD_SHAPES = {"moe_bwd_T512_train": (512, 64, 32, 8, 2, 1),
               "moe_bwd_T4096_layer": (4096, 1024, 256, 64, 8, 1)}
 F32_PEAK = 157.3e12   # MI355X fp32 vector (packed FMA)
-F32_MULADD = F32_PEAK / 4  # separate, unpacked multiply and add: 1 flop/lane/instruction
+F32_MULADD = 2 * 37.2e12  # separately rounded products and their adds, as calib_bench
+                          # measures them from registers (fp32_mfma_add_tproducts)
 
 
 def bwd_inputs(np, T, n, h, E, k, S, seed):

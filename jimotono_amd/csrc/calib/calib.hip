@@ -87,9 +87,62 @@ __global__ __launch_bounds__(512, 4) void k_issue(int iters, float *out) {
     out[blockIdx.x * 512 + threadIdx.x] = s;
 }
 
+typedef float v32f __attribute__((ext_vector_type(32)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+// The unfused and fp64 work of the backward and the exact router, by mode:
+//   9: 64 fp32 multiplies and 64 adds (16 chains of 4 pairs)
+//  10: 2 fp32 MFMAs (32x32x1, zero accumulator) and the 64 adds of their
+//      2 x 2048 products to two running sums
+//  11: 16 fp64 MFMAs (16x16x4, 4 chains of 4)
+template <int MODE>
+__global__ __launch_bounds__(512, 4) void k_products(int iters, float *out) {
+    const int lane = threadIdx.x & 63;
+    float s = 0.0f;
+    if constexpr (MODE == 9) {
+        float f[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) f[i] = lane * 0.001f + i;
+        float m = 0.999f, d = 0.001f;
+        asm volatile("" : "+v"(m), "+v"(d));  // (in registers)
+        for (int it = 0; it < iters; it++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) f[i] = __fadd_rn(__fmul_rn(f[i], m), d);
+#pragma unroll
+        for (int i = 0; i < 16; i++) s += f[i];
+    } else if constexpr (MODE == 10) {
+        const v32f zero = {};
+        v32f sum[2] = {zero, zero};
+        float a = lane * 0.001f, b = lane * 0.002f;
+        for (int it = 0; it < iters; it++)
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                asm volatile("" : "+v"(a), "+v"(b));  // (new products each time)
+                sum[r] = sum[r] + __builtin_amdgcn_mfma_f32_32x32x1f32(a, b, zero, 0, 0, 0);
+            }
+#pragma unroll
+        for (int i = 0; i < 32; i++) s += sum[0][i] + sum[1][i];
+    } else {
+        v4d acc[4] = {};
+        double a = lane * 0.001, b = lane * 0.002;
+        for (int it = 0; it < iters; it++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                acc[r % 4] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[r % 4], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) s += (float)(acc[i][0] + acc[i][3]);
+    }
+    out[blockIdx.x * 512 + threadIdx.x] = s;
+}
+
 template <int MODE>
 hipError_t launch_issue(int blocks, int iters, float *out, hipStream_t s) {
-    hipLaunchKernelGGL(k_issue<MODE>, dim3((unsigned)blocks), dim3(512), 0, s, iters, out);
+    if constexpr (MODE < 9)
+        hipLaunchKernelGGL(k_issue<MODE>, dim3((unsigned)blocks), dim3(512), 0, s, iters, out);
+    else
+        hipLaunchKernelGGL(k_products<MODE>, dim3((unsigned)blocks), dim3(512), 0, s, iters, out);
     return hipGetLastError();
 }
 
@@ -104,6 +157,9 @@ hipError_t issue_mode(int mode, int blocks, int iters, float *out, hipStream_t s
         case 6: return launch_issue<6>(blocks, iters, out, s);
         case 7: return launch_issue<7>(blocks, iters, out, s);
         case 8: return launch_issue<8>(blocks, iters, out, s);
+        case 9: return launch_issue<9>(blocks, iters, out, s);
+        case 10: return launch_issue<10>(blocks, iters, out, s);
+        case 11: return launch_issue<11>(blocks, iters, out, s);
         default: return hipErrorInvalidValue;
     }
 }
@@ -131,10 +187,10 @@ hipError_t time_launches(F f, int reps, float *ms) {
 
 }  // namespace
 
-// Mode `mode` (0-8, above) over `blocks` blocks of 8 waves, `iters`
+// Mode `mode` (0-11, above) over `blocks` blocks of 8 waves, `iters`
 // iterations per wave: *ms = mean duration of 3 timed launches.
 extern "C" int jt_calib_issue(int mode, int blocks, int iters, float *ms) {
-    if (mode < 0 || mode > 8 || blocks <= 0 || blocks > 4096 || iters <= 0 || !ms)
+    if (mode < 0 || mode > 11 || blocks <= 0 || blocks > 4096 || iters <= 0 || !ms)
         return (int)hipErrorInvalidValue;
     float *out = nullptr;
     hipError_t e = hipMalloc((void **)&out, (size_t)blocks * 512 * sizeof(float));
