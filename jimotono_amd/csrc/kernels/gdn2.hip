@@ -537,7 +537,7 @@ __device__ __forceinline__ float solve16(float x, const float4 (&m)[4], int tt) 
 // ones run: a row's M, WG, L or P values and the column's S or E values
 // (both read by 16 lanes of the wave at once). The chains are serial and
 // hold one wave per SIMD with 1024 columns on the chip, so a chunk is bound
-// by instruction latency: of 4700 cycles, phase 1 takes 2000 (128 steps of
+// by instruction latency: of 4800 cycles, phase 1 takes 2000 (128 steps of
 // two instructions, 9.7 cycles), the two solves 900, phase 3 800, LDS round
 // trips and barriers the rest. 8 heads x 4096 tokens of 128x128 in chunks of
 // 32: 256 us (with a thread per column for the solve and four barriers a

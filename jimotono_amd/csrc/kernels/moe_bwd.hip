@@ -289,8 +289,8 @@ typedef float v32f __attribute__((ext_vector_type(32)));
 // products of one k (a product of -0 comes out as +0, which changes no sum:
 // a sum that starts from +0 is never -0), the adds stay on the VALU. fp32
 // MFMA and VALU share the lanes' multipliers, so the bound is that of a
-// multiply and an add per product (147 cycles of a SIMD for 2048 measured,
-// 149 with v_mul and v_add, 33.7 T products/s on the chip). What it saves is
+// multiply and an add per product (56 ns of a SIMD for 2048 from registers,
+// with v_mul and v_add as well: 37 T products/s on the chip). What it saves is
 // everything around: one 4-byte LDS read of A and of B per lane and k for
 // 2048 products, where 4 x 4 outputs a thread read 32 bytes for 1024.
 // The two products of EPI_DUAL run one after the other.
